@@ -65,7 +65,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
            out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """x @ weight.T (+ bias).
 
-    float32 always takes the plain FMA kernel (the true 32-bit path).  bfloat16 with few rows takes the
+    float32 takes the float32 matrix-core kernel (the true 32-bit path; the plain FMA kernel where K is no multiple of 4: the
+    weight alone decides, so that every number of rows runs one of the two).  bfloat16 with few rows takes the
     hand-written few-rows MFMA kernels, with more rows the many-rows MFMA kernel (256-row tiles), whose float32
     form writes the logits of many rows without rounding them to bfloat16 (rows of an input it does not take go
     through the few-rows kernel 64 at a time).  Operands the MFMA kernels do not take (K no multiple of 8, unaligned) run the plain
@@ -73,6 +74,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     """
     out_dtype = out_dtype or x.dtype
     if x.dtype == torch.float32:
+        if out_dtype == torch.float32 and ops.linear_f32_supported(weight):
+            return ops.linear_f32(x, weight, bias)
         return ops.linear_plain(x, weight, bias, out_dtype)
     m, k = x.shape
     if k % 8 != 0 or x.data_ptr() % 16 or weight.data_ptr() % 16:

@@ -175,6 +175,33 @@ def linear_plain(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     return out
 
 
+def linear_f32_supported(weight: torch.Tensor) -> bool:
+    """Weight rows that begin on 16 bytes: what the float32 matrix-core kernel takes."""
+    return weight.shape[1] % 4 == 0 and weight.data_ptr() % 16 == 0
+
+
+def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x @ weight.T (+ bias) in float32 on the matrix cores, any number of rows.  weight: [N, K], K a multiple of 4.  An
+    element's sum has one order whatever the number of rows, so a row's result is the same bits in every launch."""
+    _need(x, "linear input", torch.float32)
+    m, k = x.shape
+    _need(weight, "linear weight", torch.float32)
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"linear: input has {k} features, weight expects {weight.shape[1]}")
+    if bias is not None:
+        _need(bias, "linear bias", torch.float32, (n,))
+        if bias.data_ptr() % 16:
+            bias = bias.clone()
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    planes = library().somi_linear_f32_planes(m, n)
+    workspace = torch.empty((planes, m, n), dtype=torch.float32, device=x.device) if planes else None
+    _check(library().somi_linear_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), _ptr(workspace), m, n, k, _stream()))
+    return out
+
+
 def linear_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                   out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """x @ weight.T (+ bias) for at most 64 bfloat16 rows on the matrix cores (weight streamed once)."""

@@ -70,6 +70,26 @@ def test_linear_plain_with_bias_and_tails(dtype, m, n, k):
         ops.linear_plain(x, rnd(n, k + 1, dtype=dtype))
 
 
+@pytest.mark.parametrize("n, k, bias", [(1, 4, True), (16, 32, False), (17, 36, True), (131, 100, False), (503, 192, True),
+                                        (896, 896, True), (4100, 68, False), (8196, 132, True)])
+def test_float32_product_on_the_matrix_cores(n, k, bias):
+    """Every kernel and tile edge against float64, and one row against the same row in every other launch, bit for bit."""
+    x, w, b = rnd(520, k, dtype="float32", seed=1), rnd(n, k, dtype="float32", seed=2), rnd(n, seed=3) if bias else None
+    exact = F.linear(x.double(), w.double(), b.double() if bias else None)
+    # a chain of K / 16 products (in units of 32), then four chains, four groups and the bias: each addition rounds once
+    bound = (math.ceil(k / 512) * 32 + 10) * 2.0 ** -24 * (F.linear(x.double().abs(), w.double().abs()) + (b.double().abs() if bias else 0))
+    whole = ops.linear_f32(x, w, b)
+    assert bool(((whole.double() - exact).abs() <= bound).all())
+    for m in (1, 2, 16, 17, 32, 33, 64, 65, 127, 129, 257):
+        assert torch.equal(ops.linear_f32(x[:m].contiguous(), w, b), whole[:m]), f"{m} rows"
+    assert torch.equal(ops.linear_f32(x[5:6].contiguous(), w, b), whole[5:6])
+    assert ops.linear_f32(x[:0].contiguous(), w, b).shape == (0, n)
+    shifted = torch.empty(3 * k + 1, device=DEV)[1:].view(3, k).copy_(x[:3])          # rows that begin off 16 bytes
+    assert torch.equal(ops.linear_f32(shifted, w, b), whole[:3])
+    with pytest.raises(KernelError, match="features"):
+        ops.linear_f32(x, rnd(n, k + 4, dtype="float32"))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("nq, nkv, d, page", [(4, 2, 16, 16), (12, 2, 48, 8), (8, 1, 80, 4), (3, 3, 128, 32)])
 def test_rope_and_cache_write(dtype, nq, nkv, d, page):

@@ -141,3 +141,11 @@ def test_the_last_columns_of_a_many_rows_product_share_k_where_whole_rounds_leav
     assert tail(1024, 37888, 3584) == (0, 1)                       # 4 x 296 = 1,184 tiles: a tail of 160
     # half the device: 1 x 296 tiles are two rounds of 128 and 40 tiles in 3 splits
     assert tail(256, 37888, 3584, units=128) == (5120, 3)
+
+
+def test_float32_products_choose_their_tiles_by_rounds_over_the_units():
+    choice = ops.library().somi_linear_f32_choice
+    assert choice(1, 151936, 256) == choice(32, 64, 256) == 0                       # few rows: the kernel that streams w
+    assert choice(33, 896, 256) == choice(512, 1152, 256) == 1 + 8                  # few tiles: their groups are shared out
+    assert choice(512, 9728, 256) == 1 and choice(64, 151936, 256) == 1             # five quarter rounds against two rounds
+    assert choice(2048, 37888, 256) == 2 and choice(33, 37888, 256) == 1            # whole rounds; rows that fill half a tile
