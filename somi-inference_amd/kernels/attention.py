@@ -56,13 +56,16 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, k_cache: torch.Tensor, v_
                     bias: torch.Tensor | None = None, score: "ops.ScoreShape | None" = None) -> torch.Tensor:
     """Attention of every token of the step over its request's cache pages -> [N, nq * D].
 
-    ``qkv`` holds each token's query heads first in its row (rotated already).  float32, and shapes the
-    MFMA kernels do not take (head sizes that are no multiple of 16, page sizes that are no multiple
-    of 4), run the plain kernel.  ``bias``: [heads, length] float32 added to the scaled scores by distance (its last
+    ``qkv`` holds each token's query heads first in its row (rotated already).  float32 has a matrix-core kernel of its
+    own; shapes the MFMA kernels do not take (head sizes that are no multiple of 16, page sizes that are no multiple
+    of 4), and float32 with biased or shaped scores, run the plain kernel.  ``bias``: [heads, length] float32 added to the scaled scores by distance (its last
     entry is 0 and stands for every key farther back).  ``score``: a cap, chunks, a sink (:class:`ops.ScoreShape`).
     """
     if score is not None and not score.any:
         score = None
+    if bias is None and score is None and ops.attention_f32_supported(qkv, k_cache):
+        return ops.attention_f32(qkv, k_cache, v_cache, block_table, step.entry_start, step.entry_first_position,
+                                 step.positions, step.max_entry_len, step.max_context, num_heads, window, scale)
     if not mfma_attention_supported(qkv, k_cache) or ((bias is not None or score is not None)
                                                       and not forms_supported(k_cache, block_table)):
         return ops.paged_attention_plain(qkv, qkv.shape[1], k_cache, v_cache, block_table,

@@ -312,6 +312,50 @@ def paged_attention_plain(q: torch.Tensor, q_stride: int, k_cache: torch.Tensor,
     return out
 
 
+def attention_f32_supported(q: torch.Tensor, k_cache: torch.Tensor) -> bool:
+    """The float32 matrix-core attention takes these heads and pages."""
+    return (q.dtype == torch.float32 and bool(library().somi_attention_f32_supported(k_cache.shape[3], k_cache.shape[2]))
+            and q.data_ptr() % 16 == 0 and q.shape[1] % 4 == 0)
+
+
+def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
+                  entry_start: torch.Tensor, entry_first: torch.Tensor, positions: torch.Tensor, max_entry_len: int,
+                  max_context: int, nq: int, window: int, scale: float, splits: int | None = None) -> torch.Tensor:
+    """Causal float32 attention of every token over its request's cached keys, on the matrix cores -> [N, nq * D].
+
+    q: [N, width], each token's query heads first in its row.  entry_start: [E + 1] offsets of the entries' tokens;
+    entry_first: [E] positions of their first tokens; max_context: the most keys that a request has.  ``splits``: how many
+    workgroups share a query's keys (None: as many as the device has room for); the result is the same bits for any."""
+    _need(q, "q", torch.float32)
+    n, width = q.shape
+    _need(k_cache, "k cache", torch.float32)
+    if k_cache.dim() != 4:
+        raise KernelError("attention_f32: the k cache must be [pages, kv_heads, page_size, head_dim]")
+    _need(v_cache, "v cache", torch.float32, _v_shape(k_cache))
+    _, nkv, page_size, head_dim = k_cache.shape
+    if width < nq * head_dim:
+        raise KernelError("attention_f32: q rows are narrower than nq * head_dim")
+    _need(block_table, "block table", torch.int32)
+    entries = block_table.shape[0]
+    _need(entry_start, "entry offsets", torch.int32, (entries + 1,))
+    _need(entry_first, "entries' first positions", torch.int32, (entries,))
+    _need(positions, "positions", torch.int32, (n,))
+    out = torch.empty((n, nq * head_dim), dtype=torch.float32, device=q.device)
+    if splits is None:
+        blocks = entries * nkv * ((max_entry_len * (nq // nkv) + 15) // 16)
+        splits = library().somi_attention_f32_splits(blocks, max_context, compute_units())
+    part_o = part_ml = None
+    if splits > 1:
+        tiles = (max_context + 63) // 64
+        part_o = torch.empty((n * nq, tiles, head_dim), dtype=torch.float32, device=q.device)
+        part_ml = torch.empty((n * nq, tiles, 2), dtype=torch.float32, device=q.device)
+    _check(library().somi_attention_f32(
+        _ptr(q), ctypes.c_int64(width), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1],
+        _ptr(entry_start), _ptr(entry_first), _ptr(positions), n, entries, int(max_entry_len), int(max_context), nq, nkv,
+        head_dim, page_size, window, ctypes.c_float(scale), int(splits), _ptr(part_o), _ptr(part_ml), _ptr(out), _stream()))
+    return out
+
+
 def attention_decode(q: torch.Tensor, q_stride: int, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      block_table: torch.Tensor, token_entry: torch.Tensor, positions: torch.Tensor,
                      nq: int, window: int, scale: float, split_len: int, num_splits: int,

@@ -179,6 +179,61 @@ def test_paged_attention_over_permuted_pages_for_portions_and_single_tokens(dtyp
     torch.testing.assert_close(out.float().view(n, nq, d).cpu(), want, **tol)
 
 
+@pytest.mark.parametrize("nq, nkv, d, page, window", [
+    (14, 2, 64, 16, 0), (28, 4, 128, 16, 0), (4, 4, 16, 4, 0), (6, 1, 32, 8, 100), (5, 5, 48, 12, 0), (20, 1, 80, 16, 70),
+    (2, 1, 256, 32, 0)])
+def test_float32_attention_on_the_matrix_cores(nq, nkv, d, page, window):
+    """Against float64, and every token's bits the same for whatever portion it arrives in and however its keys are shared
+    out.  Places of the cache that hold no key hold NaN."""
+    total = [700, 64, 1, 513]
+    n_pages = sum((t + page - 1) // page for t in total) + 2
+    perm = torch.randperm(n_pages, generator=torch.Generator().manual_seed(3)).tolist()
+    tables = [[perm.pop() for _ in range((t + page - 1) // page)] for t in total]
+    width = max(len(t) for t in tables)
+    block_table = i32([t + [0] * (width - len(t)) for t in tables])
+    kc = torch.full((n_pages, nkv, page, d), math.nan, device=DEV)
+    vc = torch.full((n_pages, nkv, d, page), math.nan, device=DEV)
+    keys = [rnd(t, nkv, d, seed=10 + i) for i, t in enumerate(total)]
+    values = [rnd(t, nkv, d, seed=20 + i) for i, t in enumerate(total)]
+    queries = [rnd(t, (nq + 1) * d, seed=30 + i, scale=2.0) for i, t in enumerate(total)]
+    for table, k, v in zip(tables, keys, values):
+        at = torch.arange(k.shape[0], device=DEV)
+        rows = torch.tensor(table, device=DEV)[at // page]
+        kc[rows, :, at % page] = k
+        vc[rows, :, :, at % page] = v
+
+    def attend(portions, splits):
+        """portions: (first, length) of each request's tokens in the step."""
+        starts = [0]
+        for _, length in portions:
+            starts.append(starts[-1] + length)
+        q = torch.cat([x[a:a + n] for x, (a, n) in zip(queries, portions)]).contiguous()
+        positions = i32([p for a, n in portions for p in range(a, a + n)])
+        out = ops.attention_f32(q, kc, vc, block_table, i32(starts), i32([a for a, _ in portions]), positions,
+                                max(n for _, n in portions), max(total) + 60, nq, window, d ** -0.5, splits)
+        return out.split([n for _, n in portions])
+
+    whole = attend([(0, t) for t in total], 1)
+    for got, q, k, v in zip(whole, queries, keys, values):
+        n = k.shape[0]
+        at = torch.arange(n, device=DEV)
+        hidden = (at > at[:, None]) | ((at <= at[:, None] - window) if window else False)
+        for h in range(nq):
+            qh, kh, vh = (x.double() for x in (q[:, h * d:(h + 1) * d], k[:, h // (nq // nkv)], v[:, h // (nq // nkv)]))
+            scores = (qh @ kh.t().contiguous() * d ** -0.5).masked_fill(hidden, -math.inf)
+            want = scores.softmax(-1) @ vh
+            # a score is off by at most d roundings of its products' size, a weight by as much relatively
+            slack = (d + 8) * 2.0 ** -24 * float(qh.norm(dim=1).max() * kh.norm(dim=1).max()) * d ** -0.5 + 600 * 2.0 ** -24
+            assert float((got[:, h * d:(h + 1) * d] - want).abs().max()) <= 2 * slack * float(vh.abs().max())
+    for portions, splits in (([(699, 1), (63, 1), (0, 1), (512, 1)], 1), ([(699, 1), (63, 1), (0, 1), (512, 1)], 5),
+                             ([(690, 8), (30, 3), (0, 1), (511, 2)], 2), ([(100, 333), (63, 1), (0, 1), (63, 65)], 1)):
+        for got, all_tokens, (a, n) in zip(attend(portions, splits), whole, portions):
+            assert torch.equal(got, all_tokens[a:a + n]), f"{portions}, {splits} splits"
+    with pytest.raises(KernelError, match="narrower"):
+        ops.attention_f32(queries[0][:, :16].contiguous(), kc, vc, block_table, i32([0] * 5), i32([0] * 4), i32([0] * 700), 1, 64, nq,
+                          window, 1.0)
+
+
 def test_paged_attention_refuses_what_it_cannot_do():
     q = rnd(1, 5 * 16)
     kc = rnd(2, 2, 4, 16)
