@@ -171,5 +171,20 @@ def load(build_if_missing: bool = True) -> ctypes.CDLL:
     return _LIB
 
 
+_PYTHON_LIB: ctypes.PyDLL | None = None
+
+
+def load_for_python() -> ctypes.PyDLL:
+    """The same library for entry points that read Python objects: calls keep the interpreter's lock and pass on the
+    exceptions they set."""
+    global _PYTHON_LIB
+    if _PYTHON_LIB is None:
+        lib = ctypes.PyDLL(load()._name)
+        lib.somi_gather_ids.argtypes = [ctypes.py_object, ctypes.c_void_p, ctypes.c_int64]
+        lib.somi_gather_ids.restype = ctypes.c_int64
+        _PYTHON_LIB = lib
+    return _PYTHON_LIB
+
+
 if __name__ == "__main__":
     print(build(force="--force" in sys.argv))

@@ -27,6 +27,10 @@ class TokenView(Sequence):
     def __init__(self, prompt: list[int], output: list[int]) -> None:
         self.prompt, self.output = prompt, output
 
+    def lists(self) -> tuple[list[int], list[int]]:
+        """What the sequence is made of, in order."""
+        return self.prompt, self.output
+
     def __len__(self) -> int:
         return len(self.prompt) + len(self.output)
 

@@ -771,17 +771,21 @@ def linear_mid(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
     return out
 
 
-def sample(logits: torch.Tensor, temperature: torch.Tensor, uniform: torch.Tensor) -> torch.Tensor:
-    """One token per row: argmax where temperature is 0, else an inverse-CDF draw from softmax(logits / T)."""
+def sample(logits: torch.Tensor, temperature: torch.Tensor, uniform: torch.Tensor,
+           cuts: torch.Tensor | None = None) -> torch.Tensor:
+    """One token per row: argmax where temperature is 0, else an inverse-CDF draw from softmax(logits / T), of the
+    entries that the row's cut (:func:`sample_cuts`) keeps."""
     _need(logits, "logits", torch.float32)
     rows, vocab = logits.shape
     _need(temperature, "temperature", torch.float32, (rows,))
     _need(uniform, "uniform", torch.float32, (rows,))
+    if cuts is not None:
+        _need(cuts, "cuts", torch.int32, (rows, 2))
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
     workspace = torch.empty((max(1, library().somi_sample_workspace_floats(rows, vocab)),), dtype=torch.float32,
                             device=logits.device)
-    _check(library().somi_sample(_ptr(logits), rows, vocab, _ptr(temperature), _ptr(uniform), _ptr(out),
-                                 _ptr(workspace), _stream()))
+    _check(library().somi_sample_through(_ptr(logits), rows, vocab, _ptr(temperature), _ptr(uniform), _ptr(cuts), _ptr(out),
+                                         _ptr(workspace), _stream()))
     return out
 
 
@@ -795,29 +799,66 @@ def repetition_penalty(logits_row: torch.Tensor, ids: torch.Tensor, penalty: flo
 
 def repetition_penalty_rows(logits: torch.Tensor, offsets: torch.Tensor, ids: torch.Tensor, penalties: torch.Tensor,
                             most_ids: int) -> None:
-    """In place on [rows, vocab] float32 logits: row r's distinct ids are ids[offsets[r]:offsets[r + 1]], its
+    """In place on [rows, vocab] float32 logits: row r's ids are ids[offsets[r]:offsets[r + 1]], its
     penalty penalties[r] (1 leaves the row alone).  ``most_ids``: the largest number of ids a row has."""
+    if most_ids < 0 or most_ids > ids.numel():
+        raise KernelError(f"repetition_penalty_rows: most_ids={most_ids} does not fit {ids.numel()} ids")
+    if most_ids:
+        penalised_rows(logits, offsets, ids, penalties, out=logits)
+
+
+def penalised_rows(logits: torch.Tensor, offsets: torch.Tensor, ids: torch.Tensor, penalties: torch.Tensor,
+                   out: torch.Tensor | None = None) -> torch.Tensor:
+    """The logits with every row's penalty on the ids it lists (each once, however often it is listed), in a tensor of
+    their own or in ``out``."""
     _need(logits, "logits", torch.float32)
     rows, vocab = logits.shape
     _need(offsets, "penalty offsets", torch.int32, (rows + 1,))
     _need(ids, "penalised ids", torch.int32)
     _need(penalties, "penalties", torch.float32, (rows,))
-    if most_ids < 0 or most_ids > ids.numel():
-        raise KernelError(f"repetition_penalty_rows: most_ids={most_ids} does not fit {ids.numel()} ids")
-    _check(library().somi_repetition_penalty_rows(_ptr(logits), rows, vocab, _ptr(offsets), _ptr(ids), _ptr(penalties),
-                                                  int(most_ids), _stream()))
+    if out is None:
+        out = torch.empty_like(logits)
+    _need(out, "penalised logits", torch.float32, (rows, vocab))
+    _check(library().somi_repetition_penalty_rows(_ptr(logits), _ptr(out), rows, vocab, _ptr(offsets), _ptr(ids),
+                                                  _ptr(penalties), _stream()))
+    return out
 
 
-def sample_filter(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor) -> None:
-    """Top-k, then top-p on softmax(logits / T), in place on [rows, vocab] float32 logits: what a rule removes
-    becomes -inf.  top_k: int32 (-1: off), top_p: float32 (1: off); rows with temperature 0 are left alone."""
+def _need_rules(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor) -> tuple[int, int]:
     _need(logits, "logits", torch.float32)
     rows, vocab = logits.shape
     _need(temperature, "temperature", torch.float32, (rows,))
     _need(top_k, "top_k", torch.int32, (rows,))
     _need(top_p, "top_p", torch.float32, (rows,))
+    return rows, vocab
+
+
+def sample_filter(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor) -> None:
+    """Top-k, then top-p on softmax(logits / T), in place on [rows, vocab] float32 logits: what a rule removes
+    becomes -inf.  top_k: int32 (-1: off), top_p: float32 (1: off); rows with temperature 0 are left alone."""
+    rows, vocab = _need_rules(logits, temperature, top_k, top_p)
     _check(library().somi_sample_filter(_ptr(logits), rows, vocab, _ptr(temperature), _ptr(top_k), _ptr(top_p),
                                         _stream()))
+
+
+def sample_cuts(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor) -> torch.Tensor:
+    """The same rules as a cut for each row, [rows, 2] int32 for :func:`sample`; the logits stay as they are."""
+    rows, vocab = _need_rules(logits, temperature, top_k, top_p)
+    cuts = torch.empty((rows, 2), dtype=torch.int32, device=logits.device)
+    _check(library().somi_sample_cuts(_ptr(logits), rows, vocab, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(cuts),
+                                      _stream()))
+    return cuts
+
+
+def gather_ids(lists: list[list[int]], out: torch.Tensor) -> int:
+    """The integers of the lists one after another into the host tensor ``out`` (int32); how many there are."""
+    if out.is_cuda or out.dtype != torch.int32 or not out.is_contiguous():
+        raise KernelError("gather_ids: the ids go to contiguous int32 host memory")
+    count = _build.load_for_python().somi_gather_ids(lists, out.data_ptr(), out.numel())
+    if count < 0:
+        raise ValueError("a token id does not fit 32 bits" if count == -2 else
+                         f"gather_ids: {sum(len(x) for x in lists)} ids for {out.numel()} places")
+    return count
 
 
 def probe_stream_shapes() -> list[str]:

@@ -4,7 +4,7 @@ Reference: ``Sampler.sample`` (somi_inference/core/sampler.py:31-55): clone,
 repetition penalty, temperature, top-k, top-p, then argmax (temperature 0) or a
 draw from the float32 softmax (:159-176).  The order and every rule are kept.
 Penalty, top-k, top-p, the temperature scaling, the softmax and the pick run in
-HIP kernels (top-k and top-p by a radix search for the cut value, without a sort).
+HIP kernels (top-k and top-p find where the row's descending order is cut, without sorting it or writing to it).
 The draw is by inverse CDF from the request's own counter-based uniform number
 instead of ``torch.multinomial`` on the global generator, so the distribution is
 the reference's and the stream is the request's own.
@@ -12,12 +12,13 @@ the reference's and the stream is the request's own.
 
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from ..kernels import ops
 from ..kernels.stages import stage
 from .params import SamplingParams
-from .rng import uniform
+from .rng import uniforms
 
 
 class PendingTokens:
@@ -51,33 +52,45 @@ class Sampler:
             events[turn[0]].synchronize()
         return ring[turn[0]], events, turn[0]
 
-    def _staged(self, values: list, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
-        """``values`` on the device through pinned memory (buffers come in power-of-two sizes, so that a few serve
-        every length)."""
-        capacity = 64
-        while capacity < len(values):
-            capacity *= 2
-        staged, events, turn = self._host_buffer("in", capacity, dtype)
-        staged[:len(values)].copy_(torch.tensor(values, dtype=dtype))
-        on_device = staged.to(device, non_blocking=True)
-        events[turn] = torch.cuda.Event()
-        events[turn].record()
-        return on_device[:len(values)]
-
-    def _row_inputs(self, plist: list[SamplingParams], seeds: list[int], counters: list[int],
-                    device: torch.device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-        """Temperatures, uniform draws, top-p values and penalties of the rows on the device, in one transfer (none
-        for all-greedy rows, which read neither of the last three)."""
+    def _row_inputs(self, plist: list[SamplingParams], histories, seeds: list[int], counters: list[int],
+                    device: torch.device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor | None]:
+        """What the rows' rules read, on the device in one transfer through pinned memory: float32 [4, rows]
+        (temperatures, uniform draws, top-p values, penalties), int32 top-k values followed by where each row's
+        penalised ids start, and the ids (None: nobody is penalised).  All-greedy rows read zeros that are kept."""
         rows = len(plist)
-        if all(p.temperature == 0.0 and p.repetition_penalty == 1.0 for p in plist):
+        penalised = [p.repetition_penalty != 1.0 and len(h) > 0 for p, h in zip(plist, histories)]
+        if not any(penalised) and all(p.temperature == 0.0 for p in plist):
             held = self._greedy_inputs.get((rows, device))
             if held is None:
-                held = self._greedy_inputs[(rows, device)] = torch.zeros(4 * rows, dtype=torch.float32, device=device)
-        else:
-            held = self._staged([p.temperature for p in plist] + [uniform(s, c) for s, c in zip(seeds, counters)]
-                                + [p.top_p for p in plist] + [p.repetition_penalty for p in plist],
-                                torch.float32, device)
-        return held[:rows], held[rows:2 * rows], held[2 * rows:3 * rows], held[3 * rows:]
+                held = self._greedy_inputs[(rows, device)] = torch.zeros(5 * rows, dtype=torch.int32, device=device)
+            return held[:4 * rows].view(torch.float32).view(4, rows), held[4 * rows:], None
+        lists, ends, total = [], [0], 0
+        for is_penalised, history in zip(penalised, histories):
+            if is_penalised:
+                parts = history.lists() if hasattr(history, "lists") else (history,)
+                lists.extend(part if type(part) is list else list(part) for part in parts)
+                total += len(history)
+            ends.append(total)
+        fixed = 6 * rows + 1
+        capacity = 64                  # buffers come in power-of-two sizes, so that a few serve every length
+        while capacity < fixed + total:
+            capacity *= 2
+        staged, events, turn = self._host_buffer("in", capacity, torch.int32)
+        words = staged.numpy()
+        floats = words[:4 * rows].view(np.float32).reshape(4, rows)
+        floats[0] = [p.temperature for p in plist]
+        floats[1] = uniforms(seeds, counters)
+        floats[2] = [p.top_p for p in plist]
+        floats[3] = [p.repetition_penalty for p in plist]
+        words[4 * rows:5 * rows] = [p.top_k for p in plist]
+        words[5 * rows:fixed] = ends
+        if total:
+            ops.gather_ids(lists, staged[fixed:fixed + total])
+        on_device = staged[:fixed + total].to(device, non_blocking=True)
+        events[turn] = torch.cuda.Event()
+        events[turn].record()
+        return (on_device[:4 * rows].view(torch.float32).view(4, rows), on_device[4 * rows:fixed],
+                on_device[fixed:] if total else None)
 
     def sample(self, logits: torch.Tensor, params: SamplingParams | list[SamplingParams],
                token_histories: list[list[int]] | None = None,
@@ -113,30 +126,16 @@ class Sampler:
             return self._draw(logits, plist, histories, seeds, counters, rows)
 
     def _draw(self, logits, plist, histories, seeds, counters, rows) -> PendingTokens:
-        needs_copy = any(p.repetition_penalty != 1.0 and h for p, h in zip(plist, histories)) or any(
-            p.temperature > 0.0 and (p.top_k != -1 or p.top_p != 1.0) for p in plist)
-        work = logits.clone() if needs_copy else logits
-        if work.dtype != torch.float32:
-            work = work.float()
+        work = logits if logits.dtype == torch.float32 else logits.float()
         work = work.contiguous()
-
-        temperature, draws, top_p, penalties = self._row_inputs(plist, seeds, counters, work.device)
-        filters = any(p.temperature > 0.0 and (p.top_k != -1 or p.top_p != 1.0) for p in plist)
-        # the rows' integers in one transfer: top-k values, then where each row's penalised ids start, then the ids
-        offsets, ids, most = [0], [], 0
-        for p, history in zip(plist, histories):
-            if p.repetition_penalty != 1.0 and history:
-                distinct = set(history)
-                ids.extend(distinct)
-                most = max(most, len(distinct))
-            offsets.append(len(ids))
-        if filters or most:
-            ints = self._staged([p.top_k for p in plist] + offsets + ids, torch.int32, work.device)
-            if most:
-                ops.repetition_penalty_rows(work, ints[rows:2 * rows + 1], ints[2 * rows + 1:], penalties, most)
-            if filters:
-                ops.sample_filter(work, temperature, ints[:rows], top_p)
-        picked = ops.sample(work, temperature, draws)
+        floats, ints, ids = self._row_inputs(plist, histories, seeds, counters, work.device)
+        temperature, draws, top_p, penalties = floats
+        cuts = None
+        if ids is not None:
+            work = ops.penalised_rows(work, ints[rows:], ids, penalties)
+        if any(p.temperature > 0.0 and (p.top_k != -1 or p.top_p != 1.0) for p in plist):
+            cuts = ops.sample_cuts(work, temperature, ints[:rows], top_p)
+        picked = ops.sample(work, temperature, draws, cuts)
         host, events, turn = self._host_buffer("out", rows, torch.int32)
         host.copy_(picked, non_blocking=True)
         copied = events[turn] = torch.cuda.Event()

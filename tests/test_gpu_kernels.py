@@ -343,6 +343,59 @@ def test_top_k_and_top_p_masks_against_the_sorted_rule(vocab):
     assert all(not math.isinf(got[row, picks[row]]) for row in range(6))
 
 
+@pytest.mark.parametrize("vocab, k, levels, skip", [(5, 3, 0, 0), (1237, 512, 0, 0), (1237, 513, 0, 1), (4096, 40, 7, 0), (30011, 700, 9, 0),
+                                                   (152064, 512, 0, 0), (152064, 64, 0, 0), (152064, 50, 4000, 4), (152064, 3000, 20, 0)])
+def test_cuts_of_rows_against_the_stable_order(vocab, k, levels, skip):
+    """Rows whose candidates fit LDS in order, and rows that fall to the search (large k, few distinct values), some of them
+    beginning off 16 bytes: the entries kept are the first of the stable descending order, the logits stay as they are, and
+    a token drawn through the cut is the token drawn from the masked row."""
+    room = rnd(6 * vocab + skip, seed=vocab % 11 + levels, scale=2.0)
+    if levels:
+        room = (room * (levels / 8)).round() / (levels / 8)
+    logits = room[skip:].view(6, vocab)
+    logits[4, 3:] = -math.inf                                # fewer finite entries than k
+    host = logits.double().cpu()
+    temps, ks, ps, kept = [0.8, 0.8, 1.3, 0.0, 1.0, 0.7], [k, k, -1, k, k, 1], [1.0, 0.0, 0.0, 0.5, 1.0, 0.9], []
+    for row in range(6):
+        order = torch.sort(host[row], descending=True, stable=True).indices
+        keep = min(ks[row], vocab) if ks[row] > 0 and temps[row] > 0 else vocab
+        if temps[row] > 0 and ps[row] < 1.0:
+            mass = torch.softmax(host[row][order[:keep]] / temps[row], -1)
+            cumulative = torch.cumsum(mass, 0)
+            if ps[row] == 0.0:                               # a p between two entries, away from rounding
+                at = min(keep // 2, 1500)
+                ps[row] = float(cumulative[at] - mass[at] / 2)
+            keep = int(((cumulative - mass) <= ps[row]).sum())
+        kept.append(order[:keep])
+    arguments = torch.tensor(temps, device=DEV), i32(ks), torch.tensor(ps, device=DEV)
+    masked, before = logits.clone(), logits.clone()
+    ops.sample_filter(masked, *arguments)
+    cuts = ops.sample_cuts(logits, *arguments)
+    assert torch.equal(logits, before)
+    for row in range(6):
+        want = torch.full((vocab,), -math.inf)
+        want[kept[row]] = before[row].cpu()[kept[row]]
+        assert torch.equal(masked[row].cpu(), want), f"row {row}: {int((masked[row].cpu() > -math.inf).sum())} kept, {len(kept[row])} expected"
+    for seed in range(5):
+        u = torch.rand(6, generator=torch.Generator().manual_seed(seed)).to(DEV)
+        assert torch.equal(ops.sample(logits, arguments[0], u, cuts), ops.sample(masked, arguments[0], u))
+
+
+@pytest.mark.parametrize("vocab, skip", [(777, 0), (8192, 0), (8192, 1), (152064, 0)])
+def test_penalised_rows_count_a_listed_id_once(vocab, skip):
+    logits = rnd(3 * vocab + skip, seed=3, scale=3.0)[skip:].view(3, vocab)
+    before = logits.clone()
+    histories = [[5, 5, vocab - 1, 5, 4095 % vocab, 4096 % vocab], [], [i * 7 % vocab for i in range(5000)]]
+    offsets = [0]
+    for history in histories:
+        offsets.append(offsets[-1] + len(history))
+    ids = i32(sum(histories, []) + [vocab])                  # (an entry past the last row's is nobody's)
+    got = ops.penalised_rows(logits, i32(offsets), ids, torch.tensor([1.7, 1.3, 0.6], device=DEV))
+    assert torch.equal(logits, before)
+    for row, penalty in enumerate([1.7, 1.3, 0.6]):
+        assert torch.equal(got[row].cpu(), plain.penalize_repetition(before[row].cpu(), histories[row], penalty)), f"row {row}"
+
+
 def test_top_k_and_top_p_masks_with_equal_entries():
     # reference test_sampler.py:96-106: exactly k survive also where the k-th value is shared
     row = torch.tensor([[5.0, 4.0, 4.0, 1.0]], device=DEV)
