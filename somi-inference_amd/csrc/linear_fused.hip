@@ -1,4 +1,4 @@
-// Two forms of the few-rows product of linear_skinny.hip (at most 64 rows) that take the RMSNorm and the
+// Two forms of the few-rows product of linear_skinny.hip (64 rows a workgroup; more rows are blocks of 64) that take the RMSNorm and the
 // residual add of a pre-norm block into the products around them, so that a decode step launches no
 // kernel of its own for either.  RMSNorm is weight * h * s with one scale s = 1 / sqrt(mean(h^2) + eps) per
 // row, and a product is linear in that scale: norm(h) . W^T = s * ((weight * h) . W^T).  So
@@ -33,6 +33,8 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 #define SOMI_BUFFER_WORD3 0x00020000u            // raw buffer, 32-bit elements, no swizzle
 #define SOMI_OUT_OF_RANGE 0x80000000u
 #define FUSED_MAX_WAVES 8
+#define FUSED_ROWS 64                            // rows of a workgroup at most
+#define FUSED_MOST_ROWS 1024                     // rows of a launch at most
 #define FUSED_CK 64
 #define FUSED_SCALED 1
 #define FUSED_RESIDUAL 2
@@ -53,7 +55,8 @@ __global__ void __launch_bounds__(FUSED_MAX_WAVES * 64)
 linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ bias,
                     TO* __restrict__ out, float* __restrict__ h, const float* __restrict__ norm_w, float eps,
                     const float* __restrict__ stats_in, int stats_blocks, int stats_stride,
-                    float* __restrict__ stats_out, bf16* __restrict__ xnext, int M, int N, int K, FusedRope rope) {
+                    float* __restrict__ stats_out, bf16* __restrict__ xnext, int M, int N, int K, int row_blocks,
+                    int column_blocks, FusedRope rope) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ float row_scale[64];
     __shared__ float part[FUSED_MAX_WAVES * 4 * 16 * MT];
@@ -64,13 +67,34 @@ linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, cons
     constexpr int NL = (NS + MT) * 2;              // loads per lane and chunk: 8 lanes read the 128 bytes of a row
     constexpr int TILES = NS * MT;
 
+    // More than 64 rows are blocks of 64.  The blocks of a column block are eight workgroups apart, so they run on one die side by side
+    // and the second finds w in that die's L2.
+    int column_block = blockIdx.x, row0 = 0;
+    if (row_blocks > 1) {
+        const int turn = blockIdx.x / (8 * row_blocks), in_turn = blockIdx.x % (8 * row_blocks);
+        column_block = turn * 8 + in_turn % 8;
+        row0 = in_turn / 8 * FUSED_ROWS;
+        if (column_block >= column_blocks) return;
+        M = min(FUSED_ROWS, M - row0);
+        x += (int64_t)row0 * K;
+        if (out) out += (int64_t)row0 * (ROPE ? rope.nq * rope.D : SWIGLU ? N / 2 : N);
+        if (h) h += (int64_t)row0 * N;
+        if (xnext) xnext += (int64_t)row0 * N;
+        if (stats_in) stats_in += row0;
+        if (stats_out) stats_out += row0;
+        if (ROPE) {
+            rope.positions += row0;
+            rope.slots += row0;
+        }
+    }
+    const int stats_here = stats_stride - row0;      // columns of the row statistics from this block's first row on
     const int waves = blockDim.x >> 6;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
     // with the rotation, workgroup b owns the columns j .. j + 15 and j + D/2 .. of head b / (D / 32)
     const int rope_blocks = ROPE ? rope.D / 32 : 1;
-    const int rope_head = blockIdx.x / rope_blocks, rope_j = (blockIdx.x % rope_blocks) * 16;
-    const int n0 = ROPE ? rope_head * rope.D + rope_j : blockIdx.x * (16 * NS);
+    const int rope_head = column_block / rope_blocks, rope_j = (column_block % rope_blocks) * 16;
+    const int n0 = ROPE ? rope_head * rope.D + rope_j : column_block * (16 * NS);
     const int strip_step = ROPE ? rope.D / 2 : 16;           // rows of w from one strip to the next
     char* mine = lds + wave * WAVE_BYTES;
 
@@ -150,7 +174,7 @@ linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, cons
     const int stats_group = wave * 4 + g, stats_groups = waves * 4;
     auto stats_load = [&](float (&to)[MT], int block) {
         const float* from = stats_in + (int64_t)block * stats_stride + r * MT;
-        if (block < stats_blocks) {
+        if (block < stats_blocks && (row_blocks == 1 || r * MT < stats_here)) {
             __builtin_memcpy(&to[0], __builtin_assume_aligned(from, MT == 3 ? 4 : 4 * MT), 4 * MT);
         } else {
 #pragma unroll
@@ -365,12 +389,12 @@ linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, cons
     }
     if (MODE == FUSED_RESIDUAL) {
         __syncthreads();
-        if (threadIdx.x < ROWS) {                    // a row's squares over the workgroup's columns, in column order
+        if (threadIdx.x < ROWS && (row_blocks == 1 || (int)threadIdx.x < stats_here)) {     // a row's squares over the workgroup's columns, in column order
             const int mt = threadIdx.x >> 4, rr = threadIdx.x & 15;
             float total = 0.f;
             for (int s = 0; s < NS; ++s)
                 for (int gg = 0; gg < 4; ++gg) total += part[(s * MT + mt) * 64 + gg * 16 + rr];
-            stats_out[(int64_t)blockIdx.x * stats_stride + threadIdx.x] = total;
+            stats_out[(int64_t)column_block * stats_stride + threadIdx.x] = total;
         }
     }
 }
@@ -391,9 +415,19 @@ static int fused_strips(int M, int N, bool swiglu) {
     return strips;
 }
 
-static int fused_waves(int K) {
+// Wavefronts that share a workgroup's K.  Eight; fewer where that leaves workgroups of the launch waiting for others: a compute unit
+// holds one or two of eight wavefronts with 64 rows (96 KB of LDS), three of four.  Measured as (8 / 4 / 2 wavefronts, us): gate_up of a 0.5B layer (304
+// workgroups, K = 896) at 16, 64 rows 8.1 / 7.5 / 8.3, 15.2 / 12.2 / 13.5, and at 128 (two blocks of 64) 22.2 / 18.2 / 15.9; q/k/v of
+// a 7B layer at 128 30.6 / 27.1 / 30.2.  One block of 16 rows over a long K streams w as fast with eight (7B gate_up 44.5 / 45.2), two
+// pay only where K is short.
+static int fused_waves(int mt, int strips, int workgroups, int K) {
     int waves = FUSED_MAX_WAVES;
     while (waves > 1 && waves * 64 > K + 63) waves /= 2;
+    const int units = somi_units();
+    const bool short_k = K <= 1024;
+    const int held = (int)(160 * 1024 / fused_lds(mt, strips, FUSED_MAX_WAVES));
+    if (waves == FUSED_MAX_WAVES && (mt > 1 ? workgroups > units * (held < 2 ? 1 : held) : short_k && workgroups > units)) waves = 4;
+    if (waves == 4 && short_k && mt == 4 && workgroups > 2 * units) waves = 2;
     return waves;
 }
 
@@ -402,15 +436,17 @@ static void fused_launch_kernel(const void* x, const void* w, const float* bias,
                                 const float* norm_w, float eps, const float* stats_in, int stats_blocks,
                                 int stats_stride, float* stats_out, void* xnext, int M, int N, int K,
                                 const FusedRope& rope, hipStream_t stream) {
-    const int waves = fused_waves(K);
-    const dim3 grid(ROPE ? (rope.nq + 2 * rope.nkv) * (rope.D / 32) : ceil_div(N, 16 * NS)), block(waves * 64);
+    const int column_blocks = ROPE ? (rope.nq + 2 * rope.nkv) * (rope.D / 32) : ceil_div(N, 16 * NS), row_blocks = ceil_div(M, FUSED_ROWS);
+    const int waves = fused_waves(MT, NS, column_blocks * row_blocks, K);
+    const dim3 grid(row_blocks > 1 ? ceil_div(column_blocks, 8) * 8 * row_blocks : column_blocks), block(waves * 64);
     const size_t smem = fused_lds(MT, NS, waves);
     if (smem > 64 * 1024)                            // beyond the default limit of dynamic LDS
         (void)hipFuncSetAttribute((const void*)linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     hipLaunchKernelGGL((linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE>), grid, block, smem, stream,
                        (const bf16*)x, (const bf16*)w, bias, (TO*)out, h, norm_w, eps, stats_in, stats_blocks,
-                       stats_stride > 0 ? stats_stride : 16 * MT, stats_out, (bf16*)xnext, M, N, K, rope);
+                       stats_stride > 0 ? stats_stride : 16 * ceil_div(M, 16), stats_out, (bf16*)xnext, M, N, K, row_blocks,
+                       column_blocks, rope);
 }
 
 template <int NS, int MODE, typename TO, bool SW, bool ROPE = false>
@@ -439,7 +475,7 @@ static int fused_launch(const void* x, const void* w, const float* bias, void* o
 
 static int fused_check(const void* x, const void* w, int M, int N, int K) {
     SOMI_REQUIRE(M >= 0 && N > 0 && K > 0, "linear_fused: bad sizes M=%d N=%d K=%d", M, N, K);
-    SOMI_REQUIRE(M <= 64, "linear_fused: at most 64 rows, got %d", M);
+    SOMI_REQUIRE(M <= FUSED_MOST_ROWS, "linear_fused: at most %d rows, got %d", FUSED_MOST_ROWS, M);
     SOMI_REQUIRE(K % 8 == 0, "linear_fused: K (%d) must be a multiple of 8", K);
     SOMI_REQUIRE((int64_t)K * 2 * 64 < (int64_t)1 << 31, "linear_fused: K (%d) is too large", K);
     SOMI_REQUIRE(((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0), "linear_fused: x and w must be 16-byte aligned");
@@ -452,7 +488,7 @@ extern "C" int somi_linear_residual_blocks(int M, int N) { return ceil_div(N, 16
 // h[m, n] += x[m, :] . w[n, :] (+ bias[n]).  x: [M, K] bfloat16; w: [N, K] bfloat16; bias: [N] float32 or null;
 // h: [M, N] float32, in and out; stats: [somi_linear_residual_blocks(M, N)][16 ceil(M / 16)] float32, out: per
 // workgroup and row the sum of squares of the new h over the workgroup's columns (rows from M on: 0); xnext:
-// [M, N] bfloat16, out, = norm_w[n] * h[m, n] (norm_w: [N] float32), or null.  M <= 64.  stats_stride: floats from
+// [M, N] bfloat16, out, = norm_w[n] * h[m, n] (norm_w: [N] float32), or null.  M <= 1,024.  stats_stride: floats from
 // one workgroup's sums to the next where they are columns of the table of more rows (a multiple of 4), or 0.
 extern "C" int somi_linear_residual(const void* x, const void* w, const float* bias, float* h, float* stats,
                                     int stats_stride, const float* norm_w, void* xnext, int M, int N, int K,
@@ -471,7 +507,7 @@ extern "C" int somi_linear_residual(const void* x, const void* w, const float* b
 // out = s * (x . w^T) (+ bias) with the row scales s[m] = 1 / sqrt(sum of stats[:, m] / K + eps), or with swiglu
 // (w: [2 I, K], gate and up rows interleaved in blocks of 16, no bias) out[m, i] = act(s g) * (s u) (swiglu 1: SiLU, 2: the tanh form of GELU) for the gate
 // and up products g, u.  x: [M, K] bfloat16, the rows a product into the stream wrote as xnext; stats:
-// [stats_blocks][16 ceil(M / 16)] float32 from the same call; out: bfloat16.  M <= 64.
+// [stats_blocks][16 ceil(M / 16)] float32 from the same call; out: bfloat16.  M <= 1,024.
 extern "C" int somi_linear_scaled(const void* x, float eps, const float* stats, int stats_blocks, const void* w,
                                   const float* bias, void* out, int M, int N, int K, int swiglu, hipStream_t stream) {
     if (fused_check(x, w, M, N, K)) return 1;
@@ -495,7 +531,7 @@ extern "C" int somi_linear_scaled(const void* x, float eps, const float* stats, 
 // first; with stats == null x is used as it is.  q: [M, nq D] bfloat16, out, rotated; k (rotated) and v go to
 // their pages: k_cache [pages, nkv, page_size, D], v_cache [pages, nkv, D, page_size], slot of row m =
 // page * page_size + offset or -1.  positions: [M] int32; inv_freq: [D / 2] float32 (the whole head is
-// rotated).  D must be a multiple of 32, M <= 64.  stats_stride: floats from one workgroup's sums to the next where
+// rotated).  D must be a multiple of 32, M <= 1,024.  stats_stride: floats from one workgroup's sums to the next where
 // the M rows are some of the rows of a longer table (a multiple of 4), or 0 for 16 ceil(M / 16).
 extern "C" int somi_linear_rope_store(const void* x, float eps, const float* stats, int stats_blocks, int stats_stride, const void* w,
                                       const float* bias, void* q, const int* positions, const int* slots,

@@ -27,6 +27,28 @@ def _mid_is_faster(m: int, n: int, k: int) -> bool:
     return (k >= LONG_K and n <= FEW_COLUMNS_PER_UNIT * units) or n >= MANY_COLUMNS_PER_UNIT * units
 
 
+FEW_ROWS = ops.FUSED_ROWS
+SMALL_PRODUCT = 4096          # 16-column strips of 64 rows times K, a compute unit: up to here blocks of 64 rows win
+NEXT_PRODUCT = 8192           # up to here with few blocks, or all at once
+
+
+def few_rows(m: int, n: int, k: int) -> bool:
+    """Whether the few-rows products that are fused with the stream and the norm take this many rows: up to 64 always, more in
+    blocks of 64 where the product is small for the device.  The many-rows kernel has 256-column tiles there that leave most
+    of the device idle, a second launch that adds the sums of its K splits and one for the rows' scales.  Measured
+    at 128 rows (many rows / blocks, us, with those launches): 0.5B q/k/v 21 / 9.5, o 16.5 / 6.2, gate_up 23 / 16, down
+    22 / 15.5; 7B q/k/v 34 / 27, o 27 / 21, but gate_up 68 / 138; at 768 rows 0.5B q/k/v 25 / 17, o 19 / 16, down
+    28 / 44.  The work of a compute unit, in strips of 16 columns by 64 rows by K, tells them apart: 0.5B down
+    loses from 5 blocks (5,320), 7B o from 3 (9,408), a 14B layer's q/k/v at once (17,920)."""
+    if m <= FEW_ROWS:
+        return True
+    blocks, strips, units = (m + FEW_ROWS - 1) // FEW_ROWS, (n + 15) // 16, ops.compute_units()
+    if m > ops.FUSED_MAX_ROWS:
+        return False
+    share = blocks * strips * k / units
+    return share <= SMALL_PRODUCT or (share <= NEXT_PRODUCT and (blocks <= 3 or blocks * strips <= units))
+
+
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, activation: str = "silu") -> torch.Tensor:
     """act(x @ gate.T) * (x @ up.T) for bfloat16 rows, act "silu" or "gelu_tanh"; weight: [2 I, K], gate and up rows
     interleaved in blocks of 16."""
@@ -41,24 +63,24 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, activation: str = "silu
 def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, h: torch.Tensor,
                     next_norm_weight: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor | None]:
     """h += x @ weight.T (+ bias) in place, by the kernel that :func:`linear` would take for the sizes; see
-    :func:`ops.linear_residual`.  More than 64 rows take the many-rows kernel, which shares a tile's K among workgroups
+    :func:`ops.linear_residual`.  Rows beyond :func:`few_rows` take the many-rows kernel, which shares a tile's K among workgroups
     where its tiles are few (o and down of 65 to some hundred rows; passes of the few-rows kernel over 64 rows each
     measured the same inside decode steps of 128 requests, 10.70 against 10.72 ms)."""
     m, n = x.shape[0], weight.shape[0]
-    if m > ops.FUSED_MAX_ROWS:
+    if not few_rows(m, n, x.shape[1]):
         return ops.linear_big_residual(x, weight, bias, h, next_norm_weight)
-    mid = _mid_is_faster(m, n, x.shape[1])
-    return ops.linear_residual(x, weight, bias, h, next_norm_weight, mid=mid)
+    mid = m <= FEW_ROWS and _mid_is_faster(m, n, x.shape[1])
+    return ops.linear_residual(x, weight, bias, h, next_norm_weight, mid=mid, row_blocks=True)
 
 
 def linear_scaled(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torch.Tensor,
                   bias: torch.Tensor | None = None, swiglu: "bool | str" = False) -> torch.Tensor:
     """The product of rows that are still to be normed, by the kernel that :func:`linear` would take for the
     sizes; see :func:`ops.linear_scaled`."""
-    if x.shape[0] > ops.FUSED_MAX_ROWS:
+    if not few_rows(x.shape[0], weight.shape[0], x.shape[1]):
         return ops.linear_big(x, weight, bias, swiglu=swiglu, eps=eps, stats=stats)
-    mid = _mid_is_faster(x.shape[0], weight.shape[0], x.shape[1])
-    return ops.linear_scaled(x, eps, stats, weight, bias, swiglu, mid=mid)
+    mid = x.shape[0] <= FEW_ROWS and _mid_is_faster(x.shape[0], weight.shape[0], x.shape[1])
+    return ops.linear_scaled(x, eps, stats, weight, bias, swiglu, mid=mid, row_blocks=True)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,

@@ -473,7 +473,14 @@ def _mid_workspace(device: torch.device) -> torch.Tensor:
     return held
 
 
-FUSED_MAX_ROWS = 64       # what the products fused with the residual add and the norm take
+FUSED_ROWS = 64           # rows that one workgroup of the products fused with the residual add and the norm takes
+FUSED_MAX_ROWS = 1024     # and, in blocks of that many, a launch
+
+
+def _need_fused_rows(m: int, row_blocks: bool) -> None:
+    most = FUSED_MAX_ROWS if row_blocks else FUSED_ROWS
+    if m > most:
+        raise KernelError(f"linear_fused: at most {most} rows, got {m}")
 
 
 def _stats_width(rows: int) -> int:
@@ -645,9 +652,10 @@ def residual_stats_blocks(m: int, n: int, k: int, mid: bool) -> int:
 
 
 def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, h: torch.Tensor,
-                    next_norm_weight: torch.Tensor | None = None, mid: bool = False
+                    next_norm_weight: torch.Tensor | None = None, mid: bool = False, row_blocks: bool = False
                     ) -> tuple[torch.Tensor, torch.Tensor | None]:
-    """h += x @ weight.T (+ bias) in float32, in place, for at most 64 bfloat16 rows.  Returns the row statistics
+    """h += x @ weight.T (+ bias) in float32, in place, for at most 64 bfloat16 rows (``row_blocks``:
+    FUSED_MAX_ROWS, in blocks of 64).  Returns the row statistics
     ``[workgroups, 16 ceil(M / 16)]`` (per workgroup and row the sum of squares of the new h over the workgroup's
     columns) and, with ``next_norm_weight``, the rows ``bfloat16(next_norm_weight * h)`` that :func:`linear_scaled`
     reads.  ``mid``: by the kernel that shares x inside a workgroup and splits K over workgroups."""
@@ -660,6 +668,7 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     if bias is not None:
         _need(bias, "linear bias", torch.float32, (n,))
     _need(h, "residual stream", torch.float32, (m, n))
+    _need_fused_rows(m, row_blocks and not mid)
     lib = library()
     blocks = residual_stats_blocks(m, n, k, mid)
     stats_stride = 0                    # rows of the statistics follow each other
@@ -680,10 +689,11 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
 
 
 def linear_scaled(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torch.Tensor,
-                  bias: torch.Tensor | None = None, swiglu: "bool | str" = False, mid: bool = False) -> torch.Tensor:
+                  bias: torch.Tensor | None = None, swiglu: "bool | str" = False, mid: bool = False,
+                  row_blocks: bool = False) -> torch.Tensor:
     """s * (x @ weight.T) (+ bias) -> bfloat16 with the row scales s = 1 / sqrt(stats.sum(0) / K + eps): the
     product of RMS-normed rows when x holds ``norm_weight * h`` and stats the sums of squares of h, both from
-    :func:`linear_residual`.  At most 64 rows.  With ``swiglu`` weight is [2 I, K] with gate and up rows
+    :func:`linear_residual`.  At most 64 rows (``row_blocks``: FUSED_MAX_ROWS).  With ``swiglu`` weight is [2 I, K] with gate and up rows
     interleaved in blocks of 16 and the result is silu(s g) * (s u) for the gate and up products g, u.
     ``mid``: by the kernel that shares x inside a workgroup and splits K over workgroups."""
     _need(x, "linear input", torch.bfloat16)
@@ -697,6 +707,7 @@ def linear_scaled(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torc
     _need(stats, "row statistics", torch.float32)
     if stats.dim() != 2 or stats.shape[1] != _stats_width(m):
         raise KernelError(f"linear_scaled: row statistics must be [blocks, {_stats_width(m)}], got {tuple(stats.shape)}")
+    _need_fused_rows(m, row_blocks and not mid)
     out = torch.empty((m, n // 2 if swiglu else n), dtype=torch.bfloat16, device=x.device)
     if mid:
         workspace = _mid_workspace(x.device)
@@ -712,14 +723,15 @@ def linear_scaled(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torc
 def linear_rope_store(x: torch.Tensor, eps: float, stats: torch.Tensor | None, weight: torch.Tensor,
                       bias: torch.Tensor | None, positions: torch.Tensor, slots: torch.Tensor, inv_freq: torch.Tensor,
                       nq: int, nkv: int, head_dim: int, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                      out: torch.Tensor | None = None) -> torch.Tensor:
-    """The q/k/v product of at most 64 bfloat16 rows with the rotary encoding of q and k and the store of k and v
+                      out: torch.Tensor | None = None, row_blocks: bool = False) -> torch.Tensor:
+    """The q/k/v product of at most 64 bfloat16 rows (``row_blocks``: FUSED_MAX_ROWS) with the rotary encoding of q and k and the store of k and v
     into their cache pages in its end -> q [M, nq * D], rotated.  weight: [(nq + 2 nkv) * D, K], q heads, k
     heads, v heads.  With ``stats`` x holds ``norm_weight * h`` and the sums are scaled per row as in
     :func:`linear_scaled` (``stats`` may be the columns of these rows in the table of more rows); without, x is
     used as it is.  The whole head is rotated (inv_freq: [D / 2]); D must be a multiple of 32."""
     _need(x, "linear input", torch.bfloat16)
     m, k = x.shape
+    _need_fused_rows(m, row_blocks)
     _need(weight, "q/k/v weight", torch.bfloat16, ((nq + 2 * nkv) * head_dim, k))
     if bias is not None:
         _need(bias, "q/k/v bias", torch.float32, (weight.shape[0],))

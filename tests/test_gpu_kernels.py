@@ -683,6 +683,51 @@ def test_products_fused_with_the_residual_add_and_the_norm(m, hidden, n_out, int
         ops.linear_residual(rnd(65, inter, dtype="bfloat16"), w1, None, rnd(65, hidden), mid=mid)
 
 
+@pytest.mark.parametrize("m, hidden, inter, nq, nkv, d", [(65, 200, 160, 3, 1, 32), (70, 896, 4864, 14, 2, 64), (129, 64, 48, 2, 2, 32),
+                                                          (200, 896, 304, 4, 4, 128), (321, 520, 1056, 6, 2, 64), (1024, 72, 32, 1, 1, 32)])
+def test_products_fused_with_the_stream_in_blocks_of_64_rows(m, hidden, inter, nq, nkv, d):
+    """Several row blocks of one launch against float32 formulas, and the q/k/v form against launches of 64 rows each."""
+    eps, page = 1e-5, 16
+    x, w1, b1 = rnd(m, inter, dtype="bfloat16", seed=1), rnd(hidden, inter, dtype="bfloat16", seed=2, scale=0.1), rnd(hidden, seed=3)
+    h, norm_w = rnd(m, hidden, seed=4, scale=2.0), 1.0 + rnd(hidden, seed=5, scale=0.1)
+    want_h = h + F.linear(x.float(), w1.float(), b1)
+    got_h = h.clone()
+    stats, weighted = ops.linear_residual(x, w1, b1, got_h, norm_w, row_blocks=True)
+    torch.testing.assert_close(got_h, want_h, atol=2e-5 * float(want_h.abs().max()) * math.sqrt(inter), rtol=1e-5)
+    width = 16 * ((m + 15) // 16)
+    assert stats.shape[1] == width and float(stats[:, m:].abs().max() if m < width else 0.0) == 0.0
+    torch.testing.assert_close(stats.sum(dim=0)[:m], got_h.pow(2).sum(dim=1), rtol=1e-5, atol=1e-6)
+    assert torch.equal(weighted, (norm_w * got_h).to(torch.bfloat16))
+
+    exact = plain_rms(got_h, norm_w, eps)
+    gate, up = rnd(inter // 16 * 16, hidden, dtype="bfloat16", seed=8, scale=0.1), rnd(inter // 16 * 16, hidden, dtype="bfloat16", seed=9, scale=0.1)
+    merged = torch.stack([gate.view(-1, 16, hidden), up.view(-1, 16, hidden)], dim=1).reshape(-1, hidden).contiguous()
+    gated = ops.linear_scaled(weighted, eps, stats, merged, swiglu=True, row_blocks=True)
+    want_gated = F.silu(exact @ gate.float().t()) * (exact @ up.float().t())
+    torch.testing.assert_close(gated.float(), want_gated, atol=float(want_gated.abs().max()) * 2 ** -5, rtol=2 ** -5)
+
+    wq, bq = rnd((nq + 2 * nkv) * d, hidden, dtype="bfloat16", seed=6, scale=0.05), rnd((nq + 2 * nkv) * d, seed=7)
+    want = F.linear(exact, wq.float(), bq)
+    scaled = ops.linear_scaled(weighted, eps, stats, wq, bq, row_blocks=True)
+    torch.testing.assert_close(scaled.float(), want, atol=float(want.abs().max()) * 2 ** -6, rtol=2 ** -6)
+    inv_freq = plain.rope_inv_freq(d, 1e4).to(DEV)
+    positions = i32([(7 * t) % 300 for t in range(m)])
+    slots = i32([-1 if t % 11 == 3 else t for t in range(m)])
+    caches = [(torch.zeros((m + page - 1) // page, nkv, page, d, dtype=torch.bfloat16, device=DEV),
+               torch.zeros((m + page - 1) // page, nkv, d, page, dtype=torch.bfloat16, device=DEV)) for _ in range(2)]
+    q = ops.linear_rope_store(weighted, eps, stats, wq, bq, positions, slots, inv_freq, nq, nkv, d, *caches[0], row_blocks=True)
+    for at in range(0, m, 64):
+        rows = slice(at, min(m, at + 64))
+        part = stats[:, at:at + 16 * ((rows.stop - at + 15) // 16)]
+        alone = ops.linear_rope_store(weighted[rows], eps, part, wq, bq, positions[rows], slots[rows], inv_freq, nq, nkv, d, *caches[1])
+        torch.testing.assert_close(q[rows].float(), alone.float(), atol=float(want.abs().max()) * 2 ** -6, rtol=2 ** -6)
+    for got, one in zip(*caches):
+        torch.testing.assert_close(got.float(), one.float(), atol=float(want.abs().max()) * 2 ** -6, rtol=2 ** -6)
+        assert torch.equal(got == 0, one == 0)
+    with pytest.raises(KernelError, match="64 rows"):
+        ops.linear_scaled(weighted, eps, stats, wq, bq)
+
+
 @pytest.mark.parametrize("m", [65, 70, 96, 128])
 @pytest.mark.parametrize("n, k", [(192, 8200), (136, 264)])
 def test_product_into_the_stream_of_65_to_128_rows(m, n, k):

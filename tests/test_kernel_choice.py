@@ -149,3 +149,12 @@ def test_float32_products_choose_their_tiles_by_rounds_over_the_units():
     assert choice(33, 896, 256) == choice(512, 1152, 256) == 1 + 8                  # few tiles: their groups are shared out
     assert choice(512, 9728, 256) == 1 and choice(64, 151936, 256) == 1             # five quarter rounds against two rounds
     assert choice(2048, 37888, 256) == 2 and choice(33, 37888, 256) == 1            # whole rounds; rows that fill half a tile
+
+
+def test_small_products_of_some_hundred_rows_run_in_blocks_of_64(device_of_256_units):
+    assert all(products.few_rows(m, 37888, 3584) for m in (1, 64)) and not products.few_rows(65, 37888, 3584)
+    assert products.few_rows(768, 1152, 896) and products.few_rows(768, 896, 896)          # a 0.5B layer's q/k/v and o
+    assert products.few_rows(256, 896, 4864) and not products.few_rows(320, 896, 4864)     # its down: five blocks are two rounds
+    assert products.few_rows(192, 9728, 896) and not products.few_rows(256, 9728, 896)
+    assert products.few_rows(128, 4608, 3584) and not products.few_rows(192, 4608, 3584)   # 7B q/k/v
+    assert not products.few_rows(1025, 16, 64)
