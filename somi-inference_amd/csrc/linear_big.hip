@@ -139,8 +139,8 @@ template <int N> __device__ __forceinline__ void big_wait_vmcnt() { asm volatile
 // to issue and their matrix instructions with them (2,048 x 37,888 x 3,584: 526 us with the burst, 457 without).
 // The wide form is persistent: a workgroup walks its die's tiles 32 apart, and the first pieces of the next
 // tile are asked for before the finished tile is stored, so the stores and the first loads overlap.
-// BM: rows of a tile, 256 (two wavefronts along m) or 128 (one: for 65 to 128 rows, where a 256-row tile would
-// spend half of its products on rows that are not there).
+// BM: rows of a tile, 256 (two wavefronts along m), 192 (two of 96 rows: five fragment reads for six products, where 128 rows have
+// six for eight) or 128 (one: for 65 to 128 rows, where a 256-row tile would spend half of its products on rows that are not there).
 // WONCE: the weight is read once (one row tile: every weight tile has a single reader), so its loads tell the caches
 // not to keep the lines, as the few-rows products' weight streams do.
 template <int BM, int BN, int S, int NW, int EPI, bool KTAIL, bool WONCE>
@@ -149,16 +149,20 @@ linear_big_kernel(const BigArgs p) {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     constexpr int BK = BIG_BK, ROW_BYTES = BIG_ROW_BYTES;
     constexpr int A_BYTES = BM * ROW_BYTES, B_BYTES = BN * ROW_BYTES, STAGE = A_BYTES + B_BYTES;
-    constexpr int WAVES_M = BM / 128, WAVES_N = NW / WAVES_M;     // wavefronts along m and along n
-    constexpr int WTM = 4, WTN = 2;                               // 32 x 32 products of a wavefront: 128 x 64
-    static_assert(BM == WAVES_M * WTM * 32 && BN / WAVES_N == WTN * 32, "a wavefront owns 128 x 64 of the tile");
+    constexpr int WAVES_M = BM == 128 ? 1 : 2, WAVES_N = NW / WAVES_M;     // wavefronts along m and along n
+    constexpr int WTM = BM / 32 / WAVES_M, WTN = 2;               // 32 x 32 products of a wavefront: 128 x 64, or 96 x 64
+    constexpr int WROWS = WTM * 32;
+    static_assert((WTM == 3 || WTM == 4) && BM == WAVES_M * WROWS && BN / WAVES_N == WTN * 32, "what a wavefront owns of the tile");
     constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, L = LA + LB;  // direct loads a lane issues per stage (8 rows each)
     constexpr int KK = BK / 16, NM = WTM * WTN, NF = WTM + WTN;
     constexpr bool HALF = S == 5;
-    static_assert(HALF || (S == 3 && L % KK == 0), "three whole stages, loads divisible over the sub-steps");
+    static_assert(HALF || S == 3, "three whole stages");
     static_assert(!HALF || (LA == LB && BN == 256 && BM == 256), "halves of equal size");
-    constexpr int LPS = HALF ? 0 : L / KK;
-    constexpr int SYNC_AFTER = 2;                                 // products of the last sub-step issued before the barrier
+    // whole stages: loads of sub-step kk and of the sub-steps before it
+    constexpr auto loads_of = [](int kk) { return (L + KK - 1 - kk) / KK; };
+    constexpr auto loads_before = [](int kk) { int sum = 0; for (int i = 0; i < kk; ++i) sum += (L + KK - 1 - i) / KK; return sum; };
+    static_assert(HALF || loads_before(KK) == L, "the sub-steps' loads are the stage's");
+    constexpr int SYNC_AFTER = NM - NF;                           // products of the last sub-step issued before the barrier
     constexpr int LSUB = HALF ? LA / KK : 1;                      // wide ring: loads of the far piece per sub-step
     static_assert(!HALF || (LA % KK == 0 && NM % LSUB == 0 && NM / LSUB > SYNC_AFTER && LA <= NF),
                   "the wide ring's loads spread over the sub-steps and the read slots");
@@ -261,7 +265,7 @@ linear_big_kernel(const BigArgs p) {
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
         const uint32_t f = frow * ROW_BYTES + (((kk * 2 + fk) ^ ((frow >> 1) & 7)) << 4);
-        foffa[kk] = lds_base + f + wm * 128 * ROW_BYTES;
+        foffa[kk] = lds_base + f + wm * WROWS * ROW_BYTES;
         foffb[kk] = lds_base + f + wn * (BN / WAVES_N) * ROW_BYTES;
     }
     // read q of a set, in the order the products need them: a[0], every b, then the other a
@@ -271,10 +275,11 @@ linear_big_kernel(const BigArgs p) {
         else if (q == 2) BIG_DS_READ(b[1], ab, 32 * ROW_BYTES);
         else if (q == 3) BIG_DS_READ(a[1], aa, 32 * ROW_BYTES);
         else if (q == 4) BIG_DS_READ(a[2], aa, 64 * ROW_BYTES);
-        else if (q == 5) BIG_DS_READ(a[3], aa, 96 * ROW_BYTES);
+        else if (WTM > 3 && q == 5) BIG_DS_READ(a[WTM - 1], aa, (WTM - 1) * 32 * ROW_BYTES);
     };
     auto wait_frags = [&](bf16x8 (&a)[WTM], bf16x8 (&b)[WTN]) {
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]));
+        if constexpr (WTM == 3) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(b[0]), "+v"(b[1]));
+        else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]));
     };
 
     // the first tile's first pieces
@@ -386,7 +391,7 @@ linear_big_kernel(const BigArgs p) {
                     for (int q = 0; q < NM; ++q) {
                         if (last && q == SYNC_AFTER) {
                             // the next stage has landed and everybody has read this one
-                            big_wait_vmcnt<(S - 3) * L + LPS * (KK - 1)>();
+                            big_wait_vmcnt<(S - 3) * L + loads_before(KK - 1)>();
                             __builtin_amdgcn_s_barrier();
                             BIG_FENCE();
                         }
@@ -395,7 +400,7 @@ linear_big_kernel(const BigArgs p) {
                         if ((!last || q >= SYNC_AFTER) && reads < NF) {
                             if (kk & 1) read_one(a0, b0, aa, ab, reads); else read_one(a1, b1, aa, ab, reads);
                             ++reads;
-                            if (loads < LPS) { issue_stage(kt + S - 1, rbuf, kk * LPS + loads); ++loads; }
+                            if (loads < loads_of(kk)) { issue_stage(kt + S - 1, rbuf, loads_before(kk) + loads); ++loads; }
                             BIG_FENCE();
                         }
                     }
@@ -415,7 +420,7 @@ linear_big_kernel(const BigArgs p) {
         if (EPI != BIG_RESIDUAL) {
 #pragma unroll
             for (int i = 0; i < WTM; ++i) {
-                const int sm = m0 + wm * 128 + i * 32 + ml;
+                const int sm = m0 + wm * WROWS + i * 32 + ml;
                 scale[i] = p.row_scale != nullptr ? p.row_scale[sm < M ? sm : M - 1] : 1.f;
             }
             if (EPI == BIG_PLAIN) {
@@ -461,7 +466,7 @@ linear_big_kernel(const BigArgs p) {
                     for (int pass = 0; pass < 4; ++pass) {
                         const int row = pass * 8 + (lane >> 3), piece = lane & 7;
                         const f32x4 v = *(const f32x4*)(stg + row * SROW + piece * 16);
-                        const int rt = wm * 128 + i * 32 + row, ct = wn * (BN / WAVES_N) + j * 32 + piece * 4;
+                        const int rt = wm * WROWS + i * 32 + row, ct = wn * (BN / WAVES_N) + j * 32 + piece * 4;
                         *(f32x4*)(slot + rt * BN + ct) = v;
                     }
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -507,7 +512,7 @@ linear_big_kernel(const BigArgs p) {
                 for (int pass = 0; pass < 32 * LPR / 64; ++pass) {
                     const int row = pass * (64 / LPR) + lane / LPR, piece = lane % LPR;
                     const u32x4 v = *(const u32x4*)(stg + row * SROW + piece * 16);
-                    const int gm = m0 + wm * 128 + i * 32 + row;
+                    const int gm = m0 + wm * WROWS + i * 32 + row;
                     const int gc = out_c0 + piece * 8;
                     if (gm < M) {
                         bf16* dst = p.out + (int64_t)gm * p.ldo + gc;
@@ -540,7 +545,7 @@ linear_big_kernel(const BigArgs p) {
                 for (int j = 0; j < WTN; ++j)
 #pragma unroll
                     for (int pass = 0; pass < 4; ++pass) {
-                        const int gm = m0 + wm * 128 + i * 32 + pass * 8 + (lane >> 3);
+                        const int gm = m0 + wm * WROWS + i * 32 + pass * 8 + (lane >> 3);
                         const int gn = wave_n0 + j * 32 + (lane & 7) * 4;
                         q[j][pass] = gm < M && gn + 4 <= N ? *(const f32x4*)(p.h + (int64_t)gm * N + gn) : f32x4{0.f, 0.f, 0.f, 0.f};
                     }
@@ -563,7 +568,7 @@ linear_big_kernel(const BigArgs p) {
                     for (int pass = 0; pass < 4; ++pass) {
                         const int row = pass * 8 + (lane >> 3), piece = lane & 7;
                         f32x4 v = *(const f32x4*)(stg + row * SROW + piece * 16);
-                        const int gm = m0 + wm * 128 + i * 32 + row;
+                        const int gm = m0 + wm * WROWS + i * 32 + row;
                         const int gn = wave_n0 + j * 32 + piece * 4;
                         if (!HALF && p.partial != nullptr) {
                             // K is split: this workgroup's sums go to its plane of the workspace as they are
@@ -610,7 +615,7 @@ linear_big_kernel(const BigArgs p) {
                         float v = sq[pass];
 #pragma unroll
                         for (int off = 4; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-                        const int gm = m0 + wm * 128 + i * 32 + pass * 8 + (lane >> 3);
+                        const int gm = m0 + wm * WROWS + i * 32 + pass * 8 + (lane >> 3);
                         if ((lane & 7) == 0 && gm < M) p.stats_out[(int64_t)stats_row * p.stats_width + gm] = v;
                     }
                 }
@@ -973,16 +978,49 @@ static bool big_streams(int tiles, int k, int cus) {
     return false;
 }
 
-// The wide tile moves fewer bytes per product and wins where it fills the device; the narrow one has twice the
-// workgroups.  Costs in units of a narrow tile's time: rounds of tiles x the tile's size (the narrow tile is
-// about 8 % less efficient per product).
-static bool big_use_wide(int m, int n, int k, int cus = 0) {
-    (void)k;
+// How many workgroups share a tile's K in the residual form (tiles of three whole stages): as many as give about
+// every compute unit a workgroup, with at least BIG_SPLIT_MIN_STAGES stages each, within the workspace; 1 where the
+// tiles alone fill half of the device.  (7B down projection at 192 rows: 28 tiles of 256 x 128, 296 stages: 227 us
+// unsplit, 62 in 9 splits.  At least 4 stages, not 8: a K of 896 has 14, and with 8 the products of a 0.5B layer at
+// 65 to 128 rows ran on the 4 or 5 workgroups of their tiles: steps of 96 / 128 requests 3.09 -> 2.63 / 3.30 -> 2.74
+// ms; at 7B sizes nothing changes.)
+#define BIG_SPLIT_MIN_STAGES 4
+static int big_splits(int tiles, int m, int n, int k, int64_t workspace_floats, int cus = 0) {
     if (cus <= 0) cus = big_compute_units();
-    const int tm = ceil_div(m, BIG_BM);
-    const double wide = (double)ceil_div(tm * ceil_div(n, 256), cus) * 2.0;
-    const double narrow = (double)ceil_div(tm * ceil_div(n, 128), cus) * 1.08;
-    return wide <= narrow;
+    const int stages = ceil_div(k, BIG_BK);
+    if (workspace_floats <= 0 || tiles * 2 > cus) return 1;
+    int64_t splits = cus / tiles;
+    if (splits > stages / BIG_SPLIT_MIN_STAGES) splits = stages / BIG_SPLIT_MIN_STAGES;
+    if (splits > workspace_floats / ((int64_t)m * n)) splits = workspace_floats / ((int64_t)m * n);
+    if (splits <= 1) return 1;
+    const int per = ceil_div(stages, (int)splits);
+    return ceil_div(stages, per);                    // no split without stages
+}
+
+// The tile of a product of more than 128 rows: 256 x 256 (returns 256), 256 x 128 (128) or 192 x 128 (192).  What a product takes is
+// whole rounds of tiles over the compute units, in units of a round of 256 x 128 tiles: a round of 256 x 256 tiles counts 1.7 and
+// one of 192 x 128 tiles 0.83 (7B gate_up, K = 3,584: 54, 92 and 45 us; 14B, K = 5,120: 76, 123 and 62), so the lower tile
+// wins where it leaves fewer rows of its last tile empty: 543 rows are 576 and not 768 (7B down 97 -> 82 us, q/k/v 39 -> 34; 14B gate_up
+// 206 -> 186).  Tiles of 128 columns share K where they are few (not in the gated form), for the planes' way to memory and back
+// (5 us and 8 bytes a value and split at 5 TB/s, beside 0.0148 us a round and value of K).  The choice depends on the sizes
+// alone, so that every caller comes to the same one.
+#define BIG_TILE_192 192
+#define BIG_COST_WIDE 1.7
+#define BIG_COST_192 0.83
+#define BIG_ASSUMED_WORKSPACE ((int64_t)34 << 20)
+static int big_choose(int m, int n, int k, bool gated, int cus = 0) {
+    if (cus <= 0) cus = big_compute_units();
+    auto rounds = [&](int rows, int columns) { return (double)ceil_div(ceil_div(m, rows) * ceil_div(n, columns), cus); };
+    auto cost = [&](int rows, double round) {
+        const int splits = gated ? 1 : big_splits(ceil_div(m, rows) * ceil_div(n, 128), m, n, k, BIG_ASSUMED_WORKSPACE, cus);
+        if (splits <= 1) return rounds(rows, 128) * round;
+        return round / splits + (5.0 + splits * 8e-6 / 5 * (double)m * n) / (0.0148 * k);
+    };
+    const double wide = rounds(256, 256) * BIG_COST_WIDE, narrow = cost(256, 1.0), low = cost(192, BIG_COST_192);
+    // (rounds that fill the device run at a lower clock, which favours the tile that moves fewer bytes: 14B down at 2,048 rows is two
+    // rounds of 192 rows, 1.66, in 326 us and one of 256 x 256, 1.7, in 304)
+    if (low < 0.97 * narrow && low < 0.95 * wide) return BIG_TILE_192;
+    return wide <= narrow ? 256 : 128;
 }
 
 // The 128-row tile: asked for (tile code BIG_TILE_LOW), or chosen for up to 128 rows.
@@ -995,7 +1033,7 @@ static bool big_use_low(int m, int tile) { return tile == BIG_TILE_LOW || (tile 
 static int big_tile_shape(int tile) { return tile % BIG_TILE_STREAM; }
 static bool big_tile_code_ok(int tile) {
     const int shape = big_tile_shape(tile);
-    return tile >= 0 && tile < 3 * BIG_TILE_STREAM && (shape == 0 || shape == BIG_TILE_LOW || shape == 128 || shape == 256);
+    return tile >= 0 && tile < 3 * BIG_TILE_STREAM && (shape == 0 || shape == BIG_TILE_LOW || shape == 128 || shape == BIG_TILE_192 || shape == 256);
 }
 
 template <int BM, int BN, int S, int NW, int EPI, bool KTAIL, bool WONCE>
@@ -1050,25 +1088,6 @@ static int big_launch_one(const BigArgs& args, hipStream_t stream) {
     else return big_launch_once<BM, BN, S, NW, EPI, KTAIL, false>(args, stream);
 }
 
-// How many workgroups share a tile's K in the residual form (tiles of three whole stages): as many as give about
-// every compute unit a workgroup, with at least BIG_SPLIT_MIN_STAGES stages each, within the workspace; 1 where the
-// tiles alone fill half of the device.  (7B down projection at 192 rows: 28 tiles of 256 x 128, 296 stages: 227 us
-// unsplit, 62 in 9 splits.  At least 4 stages, not 8: a K of 896 has 14, and with 8 the products of a 0.5B layer at
-// 65 to 128 rows ran on the 4 or 5 workgroups of their tiles: steps of 96 / 128 requests 3.09 -> 2.63 / 3.30 -> 2.74
-// ms; at 7B sizes nothing changes.)
-#define BIG_SPLIT_MIN_STAGES 4
-static int big_splits(int tiles, int m, int n, int k, int64_t workspace_floats, int cus = 0) {
-    if (cus <= 0) cus = big_compute_units();
-    const int stages = ceil_div(k, BIG_BK);
-    if (workspace_floats <= 0 || tiles * 2 > cus) return 1;
-    int64_t splits = cus / tiles;
-    if (splits > stages / BIG_SPLIT_MIN_STAGES) splits = stages / BIG_SPLIT_MIN_STAGES;
-    if (splits > workspace_floats / ((int64_t)m * n)) splits = workspace_floats / ((int64_t)m * n);
-    if (splits <= 1) return 1;
-    const int per = ceil_div(stages, (int)splits);
-    return ceil_div(stages, per);                    // no split without stages
-}
-
 template <int EPI>
 static int big_launch(BigArgs& args, int tile, hipStream_t stream, float* workspace = nullptr, int64_t workspace_floats = 0) {
     const bool ktail = args.K % BIG_BK != 0;
@@ -1101,7 +1120,15 @@ static int big_launch(BigArgs& args, int tile, hipStream_t stream, float* worksp
         stream_units(128, 256);
         return ktail ? big_launch_one<128, 256, 3, 4, EPI, true>(args, stream) : big_launch_one<128, 256, 3, 4, EPI, false>(args, stream);
     }
-    const bool wide = shape == 0 ? big_use_wide(args.M, args.N, args.K) : shape == 256;
+    const int chosen = shape == 0 ? big_choose(args.M, args.N, args.K, EPI == BIG_SWIGLU) : shape;
+    if (chosen == BIG_TILE_192) {
+        args.tiles_m = ceil_div(args.M, 192);
+        args.tiles_n = ceil_div(args.N, 128);
+        args.stats_rows = args.tiles_n * 2;
+        split_k();
+        return ktail ? big_launch_one<192, 128, 3, 4, EPI, true>(args, stream) : big_launch_one<192, 128, 3, 4, EPI, false>(args, stream);
+    }
+    const bool wide = chosen == 256;
     args.tiles_m = ceil_div(args.M, BIG_BM);
     args.tiles_n = ceil_div(args.N, wide ? 256 : 128);
     args.stats_rows = wide ? args.tiles_n * 4 : args.tiles_n * 2;
@@ -1155,14 +1182,19 @@ extern "C" int somi_row_scale(const float* stats, int blocks, int width, int m, 
     return 0;
 }
 
+// The tile that a product of more than 128 rows takes at tile code 0 (256, 192 or 128, see big_choose) on a device of `units`
+// compute units (0: the current device).
+extern "C" int somi_linear_big_choice(int m, int n, int k, int gated, int units) { return big_choose(m, n, k, gated != 0, units); }
+
 // Workgroup columns that write row statistics in the residual form: the first size of stats_out.
 // tile: 0 lets the launcher choose (the 128-row tile up to 128 rows, else 256-row tiles of the width that fills the
-// device better); 128 or 256 asks for that width of the 256-row tile, 1 for the 128-row tile (128 x 256).
+// device better, or 192 x 128); 128 or 256 asks for that width of the 256-row tile, 192 for the 192-row tile, 1 for the
+// 128-row tile (128 x 256).
 extern "C" int somi_linear_big_stats_blocks(int m, int n, int k, int tile) {
     tile = big_tile_shape(tile);
     if (big_use_low(m, tile)) return ceil_div(n, 256) * 4;
-    const bool wide = tile == 0 ? big_use_wide(m, n, k) : tile == 256;
-    return wide ? ceil_div(n, 256) * 4 : ceil_div(n, 128) * 2;
+    if (tile == 0) tile = big_choose(m, n, k, false);
+    return tile == 256 ? ceil_div(n, 256) * 4 : ceil_div(n, 128) * 2;
 }
 
 // Workgroups that share a tile's K in somi_linear_big_residual with this much workspace (1: K is not split).
@@ -1170,8 +1202,9 @@ extern "C" int somi_linear_big_splits(int m, int n, int k, int tile, int64_t wor
     if (tile - big_tile_shape(tile) == BIG_TILE_STREAM) return 1;
     tile = big_tile_shape(tile);
     if (big_use_low(m, tile)) return big_splits(ceil_div(m, 128) * ceil_div(n, 256), m, n, k, workspace_floats);
-    const bool wide = tile == 0 ? big_use_wide(m, n, k) : tile == 256;
-    return wide ? 1 : big_splits(ceil_div(m, BIG_BM) * ceil_div(n, 128), m, n, k, workspace_floats);
+    if (tile == 0) tile = big_choose(m, n, k, false);
+    if (tile == 256) return 1;
+    return big_splits(ceil_div(m, tile == BIG_TILE_192 ? 192 : BIG_BM) * ceil_div(n, 128), m, n, k, workspace_floats);
 }
 
 // Workgroups that the product's (tile, stage) units are dealt out to with this much workspace, as the entry points
@@ -1186,7 +1219,9 @@ extern "C" int somi_linear_big_streams(int m, int n, int k, int tile, int64_t wo
         bm = 128; bn = 256; tiles = ceil_div(m, 128) * ceil_div(n, 256);
         may = big_splits(tiles, m, n, k, workspace_floats) <= 1 || word == BIG_TILE_STREAM;
     } else {
-        const bool wide = shape == 0 ? big_use_wide(m, n, k, cus) : shape == 256;
+        const int chosen = shape == 0 ? big_choose(m, n, k, false, cus) : shape;
+        if (chosen == BIG_TILE_192) return 0;
+        const bool wide = chosen == 256;
         bn = wide ? 256 : 128;
         tiles = ceil_div(m, BIG_BM) * ceil_div(n, bn);
         may = wide || word == BIG_TILE_STREAM;
@@ -1223,6 +1258,9 @@ static int big_tail(int m, int n, int k, int64_t workspace_floats, int cus, int*
     const double whole_narrow = (double)ceil_div(tiles, cus);
     const double with_tail = (double)(main_cols * tiles_m) / cus + 1.0 / splits + 0.45;
     if (with_tail >= 0.97 * (whole_wide < whole_narrow ? whole_wide : whole_narrow)) return 0;
+    // the 192-row tile, by a margin: the tail's cost counts its launches in full, which run beside the rounds' end
+    const double whole_low = (double)ceil_div(ceil_div(m, 192) * col_tiles, cus) * BIG_COST_192;
+    if (1.1 * whole_low < with_tail) return 0;
     *splits_out = splits;
     return tail_n;
 }
@@ -1246,7 +1284,7 @@ extern "C" int somi_linear_big(const void* x, int64_t ldx, const void* w, int64_
     if (big_check("linear_big", x, ldx, w, ldw, m, n, k) != 0) return 1;
     SOMI_REQUIRE(out != nullptr, "linear_big: no output");
     SOMI_REQUIRE(!swiglu || (n % 32 == 0 && bias == nullptr), "linear_big: the gated form needs N a multiple of 32 and no bias");
-    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big: tile code %d (0, 1, 128 or 256, + 1000 or 2000)", tile);
+    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big: tile code %d (0, 1, 128, 192 or 256, + 1000 or 2000)", tile);
     BigArgs args = {};
     args.x = (const bf16*)x; args.ldx = ldx; args.w = (const bf16*)w; args.ldw = ldw; args.bias = bias;
     args.M = m; args.N = n; args.K = k; args.out = (bf16*)out; args.ldo = swiglu ? n / 2 : n;
@@ -1294,7 +1332,7 @@ extern "C" int somi_linear_big_residual(const void* x, int64_t ldx, const void* 
     SOMI_REQUIRE(h != nullptr, "linear_big_residual: no residual stream");
     SOMI_REQUIRE((weighted == nullptr) == (norm_w == nullptr), "linear_big_residual: the norm's weight and its rows come together");
     SOMI_REQUIRE(stats_out == nullptr || stats_width >= m, "linear_big_residual: row statistics of width %d do not cover %d rows", stats_width, m);
-    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_residual: tile code %d (0, 1, 128 or 256, + 1000 or 2000)", tile);
+    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_residual: tile code %d (0, 1, 128, 192 or 256, + 1000 or 2000)", tile);
     BigArgs args = {};
     args.x = (const bf16*)x; args.ldx = ldx; args.w = (const bf16*)w; args.ldw = ldw; args.bias = bias;
     args.M = m; args.N = n; args.K = k; args.h = h; args.norm_w = norm_w; args.weighted = (bf16*)weighted;
@@ -1311,7 +1349,7 @@ extern "C" int somi_linear_big_f32(const void* x, int64_t ldx, const void* w, in
                                    hipStream_t stream) {
     if (big_check("linear_big_f32", x, ldx, w, ldw, m, n, k) != 0) return 1;
     SOMI_REQUIRE(out != nullptr, "linear_big_f32: no output");
-    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_f32: tile code %d (0, 1, 128 or 256, + 1000 or 2000)", tile);
+    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_f32: tile code %d (0, 1, 128, 192 or 256, + 1000 or 2000)", tile);
     BigArgs args = {};
     args.x = (const bf16*)x; args.ldx = ldx; args.w = (const bf16*)w; args.ldw = ldw; args.bias = bias;
     args.M = m; args.N = n; args.K = k; args.h = out; args.overwrite = 1;
@@ -1340,7 +1378,7 @@ extern "C" int somi_linear_big_rope_store(const void* x, int64_t ldx, const void
     SOMI_REQUIRE(q && positions && slots && inv_freq && k_cache && v_cache && page_size > 0,
                  "linear_big_rope_store: q, positions, slots, inv_freq and the caches are needed");
     SOMI_REQUIRE((uintptr_t)q % 8 == 0 && (uintptr_t)k_cache % 8 == 0, "linear_big_rope_store: q and the k cache must be 8-byte aligned");
-    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_rope_store: tile code %d (0, 1, 128 or 256, + 1000 or 2000)", tile);
+    SOMI_REQUIRE(big_tile_code_ok(tile), "linear_big_rope_store: tile code %d (0, 1, 128, 192 or 256, + 1000 or 2000)", tile);
     SOMI_REQUIRE(workspace != nullptr && ((uintptr_t)workspace & 15) == 0, "linear_big_rope_store: a workspace aligned to 16 bytes is needed");
     SOMI_REQUIRE(somi_linear_big_splits(m, n, k, tile, workspace_floats) > 1,
                  "linear_big_rope_store: at m=%d n=%d k=%d the product does not share K among workgroups", m, n, k);

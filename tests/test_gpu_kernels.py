@@ -834,6 +834,31 @@ def _interleave16(gate, up):
     return torch.stack([gate.view(-1, b, h), up.view(-1, b, h)], dim=1).reshape(-1, h).contiguous()
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 130, 64), (192, 256, 200), (193, 520, 1032), (385, 96, 72), (576, 72, 8), (147, 3584, 2056),
+                                   (700, 1000, 264)])
+def test_the_192_row_tile_gives_the_bits_of_the_256_row_tile(m, n, k):
+    """Every end of the lower tile against the 256 x 128 tile, whose sums have the same order where K is not split."""
+    x, w, b = rnd(m, k, dtype="bfloat16", seed=1), rnd(n, k, dtype="bfloat16", seed=2, scale=0.1), rnd(n, seed=3)
+    norm_w, h = 1.0 + rnd(n, seed=5, scale=0.1), rnd(m, n, seed=4, scale=2.0)
+    stats = rnd(3, 16 * ((m + 15) // 16), seed=6).abs() * k
+    for arguments in (dict(), dict(bias=b), dict(bias=b, eps=1e-5, stats=stats)):
+        assert torch.equal(ops.linear_big(x, w, tile=192, split_k=False, **arguments), ops.linear_big(x, w, tile=128, split_k=False, **arguments))
+    even = w[:n // 32 * 32]
+    assert torch.equal(ops.linear_big(x, even, swiglu=True, tile=192), ops.linear_big(x, even, swiglu=True, tile=128))
+    results = []
+    for tile in (192, 128):
+        got = h.clone()
+        results.append((got, *ops.linear_big_residual(x, w, b, got, norm_w, tile=tile, split_k=False)))
+    assert all(torch.equal(a, c) for a, c in zip((results[0][0], results[0][2]), (results[1][0], results[1][2])))
+    assert torch.equal(results[0][1][:, :m], results[1][1][:, :m])
+    shared = h.clone()
+    shared_stats, _ = ops.linear_big_residual(x, w, b, shared, norm_w, tile=192)
+    torch.testing.assert_close(shared, results[0][0], atol=2e-5 * float(h.abs().max()) * math.sqrt(k), rtol=1e-5)
+    torch.testing.assert_close(shared_stats.sum(0)[:m], shared.pow(2).sum(1), rtol=1e-5, atol=1e-6)
+    got = ops.linear_big_f32(x, w, b, tile=192)
+    torch.testing.assert_close(got, F.linear(x.float(), w.float(), b), atol=2e-5 * math.sqrt(k), rtol=1e-4)
+
+
 @pytest.mark.parametrize("tile", [0, 1, 128, 256])
 @pytest.mark.parametrize("m,n,k", BIG_SHAPES)
 def test_many_rows_product_plain_with_bias_and_row_scale(m, n, k, tile):

@@ -158,3 +158,11 @@ def test_small_products_of_some_hundred_rows_run_in_blocks_of_64(device_of_256_u
     assert products.few_rows(192, 9728, 896) and not products.few_rows(256, 9728, 896)
     assert products.few_rows(128, 4608, 3584) and not products.few_rows(192, 4608, 3584)   # 7B q/k/v
     assert not products.few_rows(1025, 16, 64)
+
+
+def test_the_tile_of_a_many_rows_product_goes_with_the_rows_it_leaves_empty():
+    choice = lambda m, n, k, gated=0: ops.library().somi_linear_big_choice(m, n, k, gated, 256)
+    assert choice(2048, 37888, 3584, 1) == 256 and choice(2048, 3584, 18944) == 128            # a prompt of 7B sizes
+    assert choice(543, 27648, 5120, 1) == 192 and choice(543, 3584, 18944) == 192              # 576 rows of tiles instead of 768
+    assert choice(147, 3584, 18944) == 192 and choice(256, 3584, 18944) == 128
+    assert choice(512, 37888, 3584, 1) == 128 and choice(700, 37888, 3584, 1) == 256
