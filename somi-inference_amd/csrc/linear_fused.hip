@@ -67,15 +67,15 @@ linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, cons
     constexpr int NL = (NS + MT) * 2;              // loads per lane and chunk: 8 lanes read the 128 bytes of a row
     constexpr int TILES = NS * MT;
 
-    // More than 64 rows are blocks of 64.  The blocks of a column block are eight workgroups apart, so they run on one die side by side
+    // More rows than a workgroup takes are blocks.  The blocks of a column block are eight workgroups apart, so they run on one die side by side
     // and the second finds w in that die's L2.
     int column_block = blockIdx.x, row0 = 0;
     if (row_blocks > 1) {
         const int turn = blockIdx.x / (8 * row_blocks), in_turn = blockIdx.x % (8 * row_blocks);
         column_block = turn * 8 + in_turn % 8;
-        row0 = in_turn / 8 * FUSED_ROWS;
+        row0 = in_turn / 8 * (16 * MT);
         if (column_block >= column_blocks) return;
-        M = min(FUSED_ROWS, M - row0);
+        M = min(16 * MT, M - row0);
         x += (int64_t)row0 * K;
         if (out) out += (int64_t)row0 * (ROPE ? rope.nq * rope.D : SWIGLU ? N / 2 : N);
         if (h) h += (int64_t)row0 * N;
@@ -436,7 +436,7 @@ static void fused_launch_kernel(const void* x, const void* w, const float* bias,
                                 const float* norm_w, float eps, const float* stats_in, int stats_blocks,
                                 int stats_stride, float* stats_out, void* xnext, int M, int N, int K,
                                 const FusedRope& rope, hipStream_t stream) {
-    const int column_blocks = ROPE ? (rope.nq + 2 * rope.nkv) * (rope.D / 32) : ceil_div(N, 16 * NS), row_blocks = ceil_div(M, FUSED_ROWS);
+    const int column_blocks = ROPE ? (rope.nq + 2 * rope.nkv) * (rope.D / 32) : ceil_div(N, 16 * NS), row_blocks = ceil_div(M, 16 * MT);
     const int waves = fused_waves(MT, NS, column_blocks * row_blocks, K);
     const dim3 grid(row_blocks > 1 ? ceil_div(column_blocks, 8) * 8 * row_blocks : column_blocks), block(waves * 64);
     const size_t smem = fused_lds(MT, NS, waves);
@@ -447,6 +447,19 @@ static void fused_launch_kernel(const void* x, const void* w, const float* bias,
                        (const bf16*)x, (const bf16*)w, bias, (TO*)out, h, norm_w, eps, stats_in, stats_blocks,
                        stats_stride > 0 ? stats_stride : 16 * ceil_div(M, 16), stats_out, (bf16*)xnext, M, N, K, row_blocks,
                        column_blocks, rope);
+}
+
+// Row tiles (of 16) of a workgroup: four, or as many as there are; two or one where the blocks of 32 or 16 rows still find a compute
+// unit each, since a workgroup's time goes with its rows (0.5B layers, 64 rows a workgroup before, us: at 64 rows q/k/v
+// 9.4 -> 7.0, o 6.1 -> 4.5, down 16.0 -> 8.5; at 128 rows 9.5 -> 8.1, 6.2 -> 5.1, 15.5 -> 10.9).
+static int fused_row_tiles(int M, int column_blocks) {
+    int tiles = ceil_div(M, 16) < FUSED_ROWS / 16 ? ceil_div(M, 16) : FUSED_ROWS / 16;
+    while (tiles > 1) {
+        const int fewer = tiles > 2 ? 2 : 1;
+        if (column_blocks * ceil_div(M, 16 * fewer) > somi_units()) break;
+        tiles = fewer;
+    }
+    return tiles;
 }
 
 template <int NS, int MODE, typename TO, bool SW, bool ROPE = false>
@@ -462,7 +475,7 @@ static int fused_launch(const void* x, const void* w, const float* bias, void* o
                                                                 stats_blocks, stats_stride, stats_out, xnext, M, N,  \
                                                                 K, rope, stream);                                     \
     break
-    switch (ceil_div(M, 16)) {
+    switch (fused_row_tiles(M, ROPE ? (rope.nq + 2 * rope.nkv) * (rope.D / 32) : ceil_div(N, 16 * NS))) {
         case 1: SOMI_FUSED(1);
         case 2: SOMI_FUSED(2);
         case 3: SOMI_FUSED(3);

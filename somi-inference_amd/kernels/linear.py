@@ -36,8 +36,8 @@ def few_rows(m: int, n: int, k: int) -> bool:
     """Whether the few-rows products that are fused with the stream and the norm take this many rows: up to 64 always, more in
     blocks of 64 where the product is small for the device.  The many-rows kernel has 256-column tiles there that leave most
     of the device idle, a second launch that adds the sums of its K splits and one for the rows' scales.  Measured
-    at 128 rows (many rows / blocks, us, with those launches): 0.5B q/k/v 21 / 9.5, o 16.5 / 6.2, gate_up 23 / 16, down
-    22 / 15.5; 7B q/k/v 34 / 27, o 27 / 21, but gate_up 68 / 138; at 768 rows 0.5B q/k/v 25 / 17, o 19 / 16, down
+    at 128 rows (many rows / blocks, us, with those launches): 0.5B q/k/v 21 / 8.1, o 17 / 5.1, gate_up 23 / 16, down
+    22 / 10.9; 7B q/k/v 34 / 27, o 27 / 21, but gate_up 68 / 138; at 768 rows 0.5B q/k/v 25 / 17, o 19 / 16, down
     28 / 44.  The work of a compute unit, in strips of 16 columns by 64 rows by K, tells them apart: 0.5B down
     loses from 5 blocks (5,320), 7B o from 3 (9,408), a 14B layer's q/k/v at once (17,920)."""
     if m <= FEW_ROWS:
