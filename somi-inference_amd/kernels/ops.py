@@ -343,10 +343,11 @@ def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     out = torch.empty((n, nq * head_dim), dtype=torch.float32, device=q.device)
     if splits is None:
         blocks = entries * nkv * ((max_entry_len * (nq // nkv) + 15) // 16)
-        splits = library().somi_attention_f32_splits(blocks, max_context, compute_units())
+        splits = library().somi_attention_f32_splits(blocks, max_context, head_dim, compute_units())
     part_o = part_ml = None
     if splits > 1:
-        tiles = (max_context + 63) // 64
+        tile = library().somi_attention_f32_tile(head_dim)
+        tiles = (max_context + tile - 1) // tile
         part_o = torch.empty((n * nq, tiles, head_dim), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((n * nq, tiles, 2), dtype=torch.float32, device=q.device)
     _check(library().somi_attention_f32(
