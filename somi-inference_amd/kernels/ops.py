@@ -202,6 +202,31 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
     return out
 
 
+def linear_f32_gated_supported(weight: torch.Tensor) -> bool:
+    """The float32 product ends with silu(gate) * up for this weight ([2 I, K], gate rows first)."""
+    return linear_f32_supported(weight) and weight.shape[0] % 2 == 0 and weight.numel() * 4 < 1 << 31
+
+
+def linear_f32_gated(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate.T) * (x @ up.T) in float32 -> [M, I] for a weight [2 I, K] with the gate rows first: the bits of
+    :func:`linear_f32` followed by :func:`silu_mul`."""
+    _need(x, "linear input", torch.float32)
+    m, k = x.shape
+    _need(weight, "linear weight", torch.float32)
+    inter = weight.shape[0] // 2
+    if weight.shape[1] != k:
+        raise KernelError(f"linear: input has {k} features, weight expects {weight.shape[1]}")
+    if not linear_f32_gated_supported(weight):
+        raise KernelError(f"linear_f32_gated: a weight of {tuple(weight.shape)} is not taken")
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty((m, inter), dtype=torch.float32, device=x.device)
+    planes = library().somi_linear_f32_planes(m, 2 * inter)
+    workspace = torch.empty((planes, m, 2 * inter), dtype=torch.float32, device=x.device) if planes else None
+    _check(library().somi_linear_f32_gated(_ptr(x), _ptr(weight), _ptr(out), _ptr(workspace), m, inter, k, _stream()))
+    return out
+
+
 def linear_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                   out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """x @ weight.T (+ bias) for at most 64 bfloat16 rows on the matrix cores (weight streamed once)."""

@@ -74,6 +74,11 @@ class SwiGLU(FeedForward):
 
     def forward(self, x, step=None):
         if not self.interleaved:
+            if (self.activation == "silu" and isinstance(x, torch.Tensor) and x.dtype == torch.float32
+                    and ops.linear_f32_gated_supported(self.gate_up.weight)):
+                with stage(self.gate_up.label):
+                    gated = ops.linear_f32_gated(x, self.gate_up.weight)
+                return self.down.deferred(gated)
             projected = self.gate_up(x)                 # rows that are still to be normed are normed by the product
             with stage("activation"):
                 if self.activation == "silu":

@@ -90,6 +90,17 @@ def test_float32_product_on_the_matrix_cores(n, k, bias):
         ops.linear_f32(x, rnd(n, k + 4, dtype="float32"))
 
 
+@pytest.mark.parametrize("inter, k", [(1, 4), (16, 32), (203, 36), (520, 1000), (4864, 896), (9000, 64)])
+def test_float32_product_with_the_gate_in_its_end(inter, k):
+    """The bits of the product followed by the activation, in every kernel."""
+    x, w = rnd(1030, k, dtype="float32", seed=1), rnd(2 * inter, k, dtype="float32", seed=2, scale=0.2)
+    want = ops.silu_mul(ops.linear_f32(x, w))
+    exact = F.silu(x.double() @ w[:inter].double().t().contiguous()) * (x.double() @ w[inter:].double().t().contiguous())
+    torch.testing.assert_close(want.double(), exact, atol=1e-5 * float(exact.abs().max()), rtol=1e-4)
+    for m in (1, 16, 17, 32, 33, 64, 65, 200, 513, 1030):
+        assert torch.equal(ops.linear_f32_gated(x[:m].contiguous(), w), want[:m]), f"{m} rows"
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("nq, nkv, d, page", [(4, 2, 16, 16), (12, 2, 48, 8), (8, 1, 80, 4), (3, 3, 128, 32)])
 def test_rope_and_cache_write(dtype, nq, nkv, d, page):
