@@ -49,6 +49,28 @@ def few_rows(m: int, n: int, k: int) -> bool:
     return share <= SMALL_PRODUCT or (share <= NEXT_PRODUCT and (blocks <= 3 or blocks * strips <= units))
 
 
+EVEN_LONG_K_ROWS = 49         # from here the product with a long K into the stream takes the kernel with even shares of columns
+EVEN_WEIGHTS_PER_UNIT = 131072    # and, up to 64 rows, from this many weights a compute unit
+
+
+def even_gated(m: int, n: int, k: int) -> bool:
+    """Whether a scaled, gated product of 17 to 128 rows takes the kernel that deals its columns out evenly over the compute units:
+    where they are many for the device (37,888 columns at 17 / 64 / 128 rows 44 / 50 / 63 us against 54 / 63 / 67 of the kernels
+    below and beyond 64 rows; 17,920 16 / 20 / 25 against 18.5 / 22 / 34).  At 9,728 columns most units would have none (64 rows:
+    14.6 against 12.2), and up to 16 rows the few-rows kernel is ahead (37,888 columns, 8 rows: 44.6 against 48)."""
+    return 16 < m <= ops.EVEN_MAX_ROWS and n >= MANY_COLUMNS_PER_UNIT * ops.compute_units()
+
+
+def even_residual(m: int, n: int, k: int) -> bool:
+    """The same for the product into the stream, where K is long and the columns few: 3,584 x 18,944 at 17 / 48 / 64 / 128 rows
+    27.5 / 30.9 / 32.4 / 40 us against 26.8 / 32.0 / 35.7 / 51.  Up to 64 rows a smaller weight stays with the few-rows kernels
+    (2,048 x 11,008 at 64 rows 19.4 against 17.9, 1,536 x 8,960 17.5 against 13.9); beyond, their blocks of 64 and the many-rows
+    kernel take longer (20 and 18 against 29 and 26 at 65 rows)."""
+    units = ops.compute_units()
+    return (EVEN_LONG_K_ROWS <= m <= ops.EVEN_MAX_ROWS and k >= LONG_K and n <= FEW_COLUMNS_PER_UNIT * units
+            and (m > FEW_ROWS or n * k >= EVEN_WEIGHTS_PER_UNIT * units))
+
+
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, activation: str = "silu") -> torch.Tensor:
     """act(x @ gate.T) * (x @ up.T) for bfloat16 rows, act "silu" or "gelu_tanh"; weight: [2 I, K], gate and up rows
     interleaved in blocks of 16."""
@@ -67,6 +89,8 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     where its tiles are few (o and down of 65 to some hundred rows; passes of the few-rows kernel over 64 rows each
     measured the same inside decode steps of 128 requests, 10.70 against 10.72 ms)."""
     m, n = x.shape[0], weight.shape[0]
+    if even_residual(m, n, x.shape[1]) and ops.even_supported(x, weight, h):
+        return ops.linear_even_residual(x, weight, bias, h, next_norm_weight)
     if not few_rows(m, n, x.shape[1]):
         return ops.linear_big_residual(x, weight, bias, h, next_norm_weight)
     mid = m <= FEW_ROWS and _mid_is_faster(m, n, x.shape[1])
@@ -77,6 +101,8 @@ def linear_scaled(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torc
                   bias: torch.Tensor | None = None, swiglu: "bool | str" = False) -> torch.Tensor:
     """The product of rows that are still to be normed, by the kernel that :func:`linear` would take for the
     sizes; see :func:`ops.linear_scaled`."""
+    if swiglu and bias is None and even_gated(x.shape[0], weight.shape[0], x.shape[1]) and ops.even_supported(x, weight, stats):
+        return ops.linear_even_gated(x, eps, stats, weight, swiglu)
     if not few_rows(x.shape[0], weight.shape[0], x.shape[1]):
         return ops.linear_big(x, weight, bias, swiglu=swiglu, eps=eps, stats=stats)
     mid = x.shape[0] <= FEW_ROWS and _mid_is_faster(x.shape[0], weight.shape[0], x.shape[1])

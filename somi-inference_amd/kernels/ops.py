@@ -788,6 +788,59 @@ def linear_rope_store(x: torch.Tensor, eps: float, stats: torch.Tensor | None, w
     return q
 
 
+EVEN_MAX_ROWS = 128       # what the product with its columns dealt out evenly takes
+
+
+def even_supported(x: torch.Tensor, weight: torch.Tensor, *others: torch.Tensor) -> bool:
+    """Whether :func:`linear_even_gated` and :func:`linear_even_residual` take these operands (others: h or the statistics)."""
+    return (x.shape[0] <= EVEN_MAX_ROWS and x.shape[1] % 8 == 0
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, weight, *others)))
+
+
+def _even_operands(x: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int]:
+    _need(x, "linear input", torch.bfloat16)
+    m, k = x.shape
+    _need(weight, "linear weight", torch.bfloat16)
+    if weight.shape[1] != k:
+        raise KernelError(f"linear: input has {k} features, weight expects {weight.shape[1]}")
+    return m, weight.shape[0], k
+
+
+def linear_even_gated(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torch.Tensor,
+                      swiglu: "bool | str" = True) -> torch.Tensor:
+    """:func:`linear_scaled`'s gated form for at most 128 rows, by the kernel that deals the columns out evenly over the
+    compute units: act(s g) * (s u) -> bfloat16 [M, I], weight [2 I, K] with gate and up rows interleaved in blocks of 16."""
+    m, n, k = _even_operands(x, weight)
+    if n % 32:
+        raise KernelError(f"linear_scaled: weight {tuple(weight.shape)} does not hold pairs of 16 gate and up rows")
+    _need(stats, "row statistics", torch.float32)
+    if stats.dim() != 2 or stats.shape[1] != _stats_width(m):
+        raise KernelError(f"linear_scaled: row statistics must be [blocks, {_stats_width(m)}], got {tuple(stats.shape)}")
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+    _check(library().somi_linear_even_gated(_ptr(x), ctypes.c_float(eps), _ptr(stats), stats.shape[0], stats.shape[1], _ptr(weight),
+                                            _ptr(out), m, n, k, gate_code(swiglu), _stream()))
+    return out
+
+
+def linear_even_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, h: torch.Tensor,
+                         next_norm_weight: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """:func:`linear_residual` for at most 128 rows, by the kernel that deals the columns, and K where they are few, out evenly over
+    the compute units."""
+    m, n, k = _even_operands(x, weight)
+    if bias is not None:
+        _need(bias, "linear bias", torch.float32, (n,))
+    _need(h, "residual stream", torch.float32, (m, n))
+    stats = torch.empty(((n + 63) // 64, _stats_width(m)), dtype=torch.float32, device=x.device)
+    weighted = None
+    if next_norm_weight is not None:
+        _need(next_norm_weight, "norm weight", torch.float32, (n,))
+        weighted = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    planes = torch.empty((library().somi_linear_even_planes(n, k), m, n), dtype=torch.float32, device=x.device)
+    _check(library().somi_linear_even_residual(_ptr(x), _ptr(weight), _ptr(bias), _ptr(h), _ptr(stats), stats.shape[1],
+                                               _ptr(next_norm_weight), _ptr(weighted), _ptr(planes), m, n, k, _stream()))
+    return stats, weighted
+
+
 def linear_mid(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                out_dtype: torch.dtype | None = None, swiglu: "bool | str" = False) -> torch.Tensor:
     """x @ weight.T (+ bias) for at most 64 bfloat16 rows, x shared by the wavefronts of a workgroup, K split

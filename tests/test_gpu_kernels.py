@@ -762,6 +762,43 @@ def test_product_into_the_stream_of_65_to_128_rows(m, n, k):
     torch.testing.assert_close(got.float(), want, atol=float(want.abs().max()) * 2 ** -6, rtol=2 ** -6)
 
 
+@pytest.mark.parametrize("m, n, k, act", [(17, 32, 8, "silu"), (1, 96, 72, "silu"), (33, 24576, 64, "gelu_tanh"), (64, 27648 - 32, 136, "silu"),
+                                          (32, 37888, 328, "silu"), (65, 37888 + 32, 72, "silu"), (128, 36864, 256, "gelu_tanh"),
+                                          (50, 160, 2048, "silu"), (128, 24576 + 64, 4096, "silu")])
+def test_gated_product_with_its_columns_dealt_out_evenly(m, n, k, act):
+    """Each number of strips and of row tiles, columns and K that end inside a workgroup and a stage, and rows 4 KB apart (whose
+    workgroups start at different stages) against the float32 formula."""
+    x, w = rnd(m, k, dtype="bfloat16", seed=1), rnd(n, k, dtype="bfloat16", seed=2, scale=0.1)
+    width = 16 * ((m + 15) // 16)
+    stats = rnd(5, width, seed=3).abs() * k
+    scale = torch.rsqrt(stats[:, :m].sum(dim=0) / k + 1e-5)[:, None]
+    both = (scale * (x.float() @ w.float().t())).view(m, n // 32, 2, 16)
+    gate, up = both[:, :, 0].reshape(m, -1), both[:, :, 1].reshape(m, -1)
+    want = (F.silu(gate) if act == "silu" else F.gelu(gate, approximate="tanh")) * up
+    got = ops.linear_even_gated(x, 1e-5, stats, w, act)
+    # the result's own rounding, 2^-9, and float32 sums in another order: far below 2^-12 of the largest
+    torch.testing.assert_close(got.float(), want, rtol=2 ** -8, atol=float(want.abs().max()) * 2 ** -12)
+    with pytest.raises(KernelError, match="row statistics"):
+        ops.linear_even_gated(x, 1e-5, stats[:, :m - 1], w, act)
+
+
+@pytest.mark.parametrize("m, n, k", [(49, 128, 8192), (64, 3584, 18944), (65, 1000, 8200), (128, 130, 264), (100, 33, 8), (1, 5120, 520)])
+def test_product_into_the_stream_with_even_shares_of_columns(m, n, k):
+    x, w, b = rnd(m, k, dtype="bfloat16", seed=1), rnd(n, k, dtype="bfloat16", seed=2, scale=0.1), rnd(n, seed=3)
+    h, norm_w = rnd(m, n, seed=4, scale=2.0), 1.0 + rnd(n, seed=5, scale=0.1)
+    want_h = h + F.linear(x.float(), w.float(), b)
+    got_h = h.clone()
+    stats, weighted = ops.linear_even_residual(x, w, b, got_h, norm_w)
+    torch.testing.assert_close(got_h, want_h, atol=2e-5 * float(want_h.abs().max()) * math.sqrt(k), rtol=1e-5)
+    width = 16 * ((m + 15) // 16)
+    assert stats.shape == ((n + 63) // 64, width) and float(stats[:, m:].abs().max() if m < width else 0.0) == 0.0
+    torch.testing.assert_close(stats.sum(dim=0)[:m], got_h.pow(2).sum(dim=1), rtol=1e-5, atol=1e-6)
+    assert torch.equal(weighted, (norm_w * got_h).to(torch.bfloat16))
+    alone = h.clone()
+    assert ops.linear_even_residual(x, w, None, alone)[1] is None
+    torch.testing.assert_close(alone, want_h - b, atol=2e-5 * float(want_h.abs().max()) * math.sqrt(k), rtol=1e-5)
+
+
 @pytest.mark.parametrize("scaled", [True, False], ids=["normed", "as-is"])
 @pytest.mark.parametrize("m, nq, nkv, d, hidden, page", [(1, 4, 2, 32, 64, 16), (9, 12, 2, 64, 200, 8), (16, 3, 3, 128, 520, 4),
                                                          (24, 6, 2, 96, 264, 8), (37, 5, 1, 96, 1000, 16), (64, 28, 4, 128, 3584, 16)])

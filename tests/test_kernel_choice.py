@@ -166,3 +166,25 @@ def test_the_tile_of_a_many_rows_product_goes_with_the_rows_it_leaves_empty():
     assert choice(543, 27648, 5120, 1) == 192 and choice(543, 3584, 18944) == 192              # 576 rows of tiles instead of 768
     assert choice(147, 3584, 18944) == 192 and choice(256, 3584, 18944) == 128
     assert choice(512, 37888, 3584, 1) == 128 and choice(700, 37888, 3584, 1) == 256
+
+
+def test_even_shares_of_columns(monkeypatch):
+    import ctypes
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    strips, splits = ctypes.c_int(), ctypes.c_int()
+
+    def shape(m, n, k, units=256):
+        assert ops.library().somi_linear_even_choice(m, n, k, units, ctypes.byref(strips), ctypes.byref(splits)) == 0
+        return strips.value, splits.value
+
+    assert [shape(m, 37888, 3584)[0] for m in (17, 64, 128)] == [10, 12, 12]         # 237 workgroups; 198, which read x less often
+    assert shape(64, 27648, 5120)[0] == 8 and shape(64, 22016, 4096)[0] == 6          # 216, 230
+    assert shape(64, 3584, 18944)[1] == 9 and shape(64, 5120, 13824)[1] == 6          # 28 x 9 and 40 x 6 workgroups
+    for n, k in ((16, 8), (130, 264), (8192, 8192), (3584, 18944), (1000, 70000)):    # every split has a stage
+        count, stages = shape(64, n, k)[1], (k + 63) // 64
+        assert count >= 1 and (count - 1) * ((stages + count - 1) // count) < stages
+    assert products.even_gated(17, 37888, 3584) and products.even_gated(128, 17920, 1536)
+    assert not any(products.even_gated(m, 37888, 3584) for m in (1, 16, 129)) and not products.even_gated(64, 9728, 896)
+    assert products.even_residual(49, 3584, 18944) and not products.even_residual(48, 3584, 18944)
+    assert not products.even_residual(64, 1536, 8960) and products.even_residual(128, 1536, 8960)
+    assert not products.even_residual(129, 3584, 18944) and not products.even_residual(128, 3584, 3584)
