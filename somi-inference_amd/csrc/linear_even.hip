@@ -1,4 +1,4 @@
-// The product of some tens of rows (17 to 128) with its columns dealt out evenly over the compute units: bfloat16 in, float32 sums on
+// The product of some tens of rows (17 to 192) with its columns dealt out evenly over the compute units: bfloat16 in, float32 sums on
 // the matrix cores.
 //
 // Reference: the same nn.Linear products as linear_plain.hip (somi_inference/models/qwen2.py:221-222, 268-271;
@@ -9,13 +9,13 @@
 // gate_up, 37,888 x 3,584, at 64 rows: 592 workgroups on 256 units, 57 us and a reduce of 8, where the weight alone takes 41); 256-column
 // tiles of the many-rows kernel leave 108 of 256 units without one (71 us at 128 rows).  Here a workgroup has a compute unit
 // to itself and owns NS strips of 16 columns over all of K.  Measured, the launches that it replaces / here, us at 17, 64 and 128 rows:
-//   gate_up of 37,888 x 3,584: 54 / 44, 63 / 50, 67 / 63;  of 27,648 x 5,120: 57 / 48, 65 / 55, 91 / 68;
-//   of 28,672 x 4,096: 57 / 39, 58 / 41, 71 / 50 (see the start of a workgroup's K below);
-//   down of 3,584 x 18,944: 27 / 28, 36 / 32, 51 / 40;  of 5,120 x 13,824: 28 / 29, 35 / 33, 50 / 40.
+//   gate_up of 37,888 x 3,584: 55 / 45, 63 / 51, 68 / 63 (at 192 rows 86 / 77);  of 27,648 x 5,120: 57 / 49, 65 / 56, 90 / 69;
+//   of 28,672 x 4,096: 62 / 37, 61 / 40, 72 / 50 (see the start of a workgroup's K below);
+//   down of 3,584 x 18,944: 27 / 28, 35 / 32, 50 / 39;  of 5,120 x 13,824: 28 / 30, 34 / 33, 50 / 40.
 // What is left above the weight's time is x, which every workgroup reads: 7 TB/s of w and x together.
 //
 // Eight wavefronts share a stage (64 values of K: one 128-byte line of each of the workgroup's rows of w and of x) through LDS,
-// held twice; the next DEPTH stages are on their way in registers.  Wavefront v owns row tiles v % 4 (and v % 4 + 4) and a share
+// held twice; the next DEPTH stages are on their way in registers.  Wavefront v owns row tiles v % 4 (v % 4 + 4, v % 4 + 8) and a share
 // of the strips, by pairs (a gate strip and its up strip).  w is the A operand, so a lane has four neighbouring columns of a row.
 #include "common.h"
 
@@ -29,7 +29,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 #define EVEN_THREADS 512
 #define EVEN_CK 64                                // values of K of a stage
 #define EVEN_DEPTH 4
-#define EVEN_MOST_ROWS 128
+#define EVEN_MOST_ROWS 192
 
 enum EvenForm { EVEN_GATED = 0, EVEN_PLANES = 1 };
 
@@ -55,7 +55,7 @@ linear_even_kernel(const EvenArgs p) {
     constexpr int RPW = RT > 4 ? RT / 4 : 1;              // row tiles of a wavefront
     constexpr int ROW_GROUPS = RT > 4 ? 4 : RT, STRIP_GROUPS = 8 / ROW_GROUPS, PAIRS = NS / 2;
     constexpr int MOST = 2 * ((PAIRS + STRIP_GROUPS - 1) / STRIP_GROUPS);      // strips of a wavefront at most
-    static_assert(NS % 2 == 0 && (RT == 2 || RT == 4 || RT == 8), "pairs of strips, 32, 64 or 128 rows");
+    static_assert(NS % 2 == 0 && (RT == 2 || RT == 4 || RT == 8 || RT == 12), "pairs of strips, 32, 64, 128 or 192 rows");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     float* part = reinterpret_cast<float*>(lds + 2 * STAGE);     // [EVEN_THREADS] parts of the rows' sums of squares
     float* scale = part + EVEN_THREADS;                          // [ROWS]
@@ -138,7 +138,7 @@ linear_even_kernel(const EvenArgs p) {
         constexpr int E = EVEN_THREADS / ROWS;
         const int row = tid % ROWS, e = tid / ROWS;
         float sum = 0.f;
-        if (row < M)
+        if (row < M && e < E)
             for (int b = e; b < p.stats_blocks; b += E) sum += p.stats[(int64_t)b * p.stats_stride + row];
         part[tid] = sum;
         __syncthreads();
@@ -249,7 +249,7 @@ linear_even_stream_kernel(const float* __restrict__ planes, int splits, const fl
 // the time of the lines that each reads, and no less than what four fifths of the units read at the memory's rate (37,888 x 3,584: at 64 rows 8 / 10 / 12
 // strips 71 / 53 / 50 to 55 us, at 128 88 / 66 / 62; 27,648 x 5,120 at 64 rows 57 / 75 / 67).
 static int even_strips(int M, int N, int units) {
-    const int strips = ceil_div(N, 16), rows = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+    const int strips = ceil_div(N, 16), rows = ceil_div(M, 16) * 16;
     int64_t best = -1;
     int chosen = 0;
     for (int ns = 6; ns <= 12; ns += 2) {
@@ -303,7 +303,7 @@ static int even_launch(const EvenArgs& a, hipStream_t stream) {
 
 // out[m, i] = act(s g) * (s u) -> bfloat16 [M, N / 2] for the products g, u of x's rows with w's gate and up rows (interleaved in
 // blocks of 16); s[m] = 1 / sqrt(sum of stats[:, m] / K + eps) with stats [stats_blocks][stats_stride >= M] partial sums of squares.
-// act 1: SiLU, 2: the tanh form of GELU.  M <= 128, N a multiple of 32, out 8-byte aligned.
+// act 1: SiLU, 2: the tanh form of GELU.  M <= 192, N a multiple of 32, out 8-byte aligned.
 extern "C" int somi_linear_even_gated(const void* x, float eps, const float* stats, int stats_blocks, int stats_stride, const void* w,
                                       void* out, int M, int N, int K, int act, hipStream_t stream) {
     if (even_check(x, w, M, N, K)) return 1;
@@ -322,7 +322,8 @@ extern "C" int somi_linear_even_gated(const void* x, float eps, const float* sta
                           : even_launch<RT, 12, EVEN_GATED>(a, stream)
     if (M <= 32) SOMI_EVEN(2);
     if (M <= 64) SOMI_EVEN(4);
-    SOMI_EVEN(8);
+    if (M <= 128) SOMI_EVEN(8);
+    SOMI_EVEN(12);
 #undef SOMI_EVEN
 }
 
@@ -331,10 +332,11 @@ extern "C" int somi_linear_even_planes(int N, int K) { return N > 0 && K > 0 ? e
 
 // h[m, n] += x[m, :] . w[n, :] (+ bias[n]), float32 in place; planes: somi_linear_even_planes(N, K) planes of [M, N] float32; stats:
 // [ceil(N / 64)][stats_stride >= M], out, sums of squares of the new h over 64 columns each (0 from M on); weighted: [M, N] bfloat16 =
-// norm_w * h, or null.  M <= 128; planes and h 16-byte, weighted 8-byte aligned.
+// norm_w * h, or null.  M <= 128 rows; planes and h 16-byte, weighted 8-byte aligned.
 extern "C" int somi_linear_even_residual(const void* x, const void* w, const float* bias, float* h, float* stats, int stats_stride,
                                          const float* norm_w, void* weighted, float* planes, int M, int N, int K, hipStream_t stream) {
     if (even_check(x, w, M, N, K)) return 1;
+    SOMI_REQUIRE(M <= 128, "linear_even: at most 128 rows into the stream, got %d", M);
     SOMI_REQUIRE(h && stats && planes && stats_stride >= M, "linear_even: h, stats and the planes are needed");
     SOMI_REQUIRE(!weighted || norm_w, "linear_even: the next rows need the norm's weight");
     SOMI_REQUIRE((((uintptr_t)h | (uintptr_t)planes) & 15) == 0 && (uintptr_t)weighted % 8 == 0, "linear_even: h and the planes must be aligned");

@@ -49,16 +49,24 @@ def few_rows(m: int, n: int, k: int) -> bool:
     return share <= SMALL_PRODUCT or (share <= NEXT_PRODUCT and (blocks <= 3 or blocks * strips <= units))
 
 
+EVEN_COLUMNS_PER_UNIT = 192   # the widest workgroup of the kernel that deals columns out evenly
 EVEN_LONG_K_ROWS = 49         # from here the product with a long K into the stream takes the kernel with even shares of columns
 EVEN_WEIGHTS_PER_UNIT = 131072    # and, up to 64 rows, from this many weights a compute unit
 
 
 def even_gated(m: int, n: int, k: int) -> bool:
-    """Whether a scaled, gated product of 17 to 128 rows takes the kernel that deals its columns out evenly over the compute units:
-    where they are many for the device (37,888 columns at 17 / 64 / 128 rows 44 / 50 / 63 us against 54 / 63 / 67 of the kernels
-    below and beyond 64 rows; 17,920 16 / 20 / 25 against 18.5 / 22 / 34).  At 9,728 columns most units would have none (64 rows:
-    14.6 against 12.2), and up to 16 rows the few-rows kernel is ahead (37,888 columns, 8 rows: 44.6 against 48)."""
-    return 16 < m <= ops.EVEN_MAX_ROWS and n >= MANY_COLUMNS_PER_UNIT * ops.compute_units()
+    """Whether a scaled, gated product of 17 to 192 rows takes the kernel that deals its columns out evenly over the compute units:
+    where they are more than 64 a unit and fit into one round of its workgroups, of up to 192 columns (37,888 columns at
+    17 / 64 / 128 rows 45 / 51 / 63 us against 55 / 63 / 68 of the kernels below and beyond 64 rows; 17,920 15 / 21 / 25 against
+    18 / 23 / 34).  16,384 columns are one whole round of the kernel that splits K (64 rows: 31 against 27), fewer leave units
+    without a workgroup, and up to 16 rows the few-rows kernel is ahead (37,888 columns, 8 rows: 44.6 against 48).  In two
+    rounds it is ahead only up to 64 rows with inputs a multiple of 4 KB (57,344 x 8,192 at 64 rows 156 against 195; at 128 rows 182
+    against 160; 55,296 x 5,120 at 64 rows 111 against 106).  Beyond 128 rows the many-rows kernel's 192-row tiles of 128 columns
+    are ahead as long as they are one round (27,648 columns at 160 rows 79 against 82; 37,888 86 against 73)."""
+    per_unit = n / ops.compute_units()
+    if m <= 16 or m > ops.EVEN_MAX_ROWS or per_unit <= (MANY_COLUMNS_PER_UNIT if m <= 128 else 2 * MANY_COLUMNS_PER_UNIT):
+        return False
+    return per_unit <= EVEN_COLUMNS_PER_UNIT or (m <= FEW_ROWS and k % 2048 == 0)
 
 
 def even_residual(m: int, n: int, k: int) -> bool:
@@ -67,7 +75,7 @@ def even_residual(m: int, n: int, k: int) -> bool:
     (2,048 x 11,008 at 64 rows 19.4 against 17.9, 1,536 x 8,960 17.5 against 13.9); beyond, their blocks of 64 and the many-rows
     kernel take longer (20 and 18 against 29 and 26 at 65 rows)."""
     units = ops.compute_units()
-    return (EVEN_LONG_K_ROWS <= m <= ops.EVEN_MAX_ROWS and k >= LONG_K and n <= FEW_COLUMNS_PER_UNIT * units
+    return (EVEN_LONG_K_ROWS <= m <= 128 and k >= LONG_K and n <= FEW_COLUMNS_PER_UNIT * units
             and (m > FEW_ROWS or n * k >= EVEN_WEIGHTS_PER_UNIT * units))
 
 

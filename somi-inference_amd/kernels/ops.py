@@ -788,7 +788,7 @@ def linear_rope_store(x: torch.Tensor, eps: float, stats: torch.Tensor | None, w
     return q
 
 
-EVEN_MAX_ROWS = 128       # what the product with its columns dealt out evenly takes
+EVEN_MAX_ROWS = 192       # what the gated product with its columns dealt out evenly takes; into the stream 128
 
 
 def even_supported(x: torch.Tensor, weight: torch.Tensor, *others: torch.Tensor) -> bool:
@@ -808,7 +808,7 @@ def _even_operands(x: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int
 
 def linear_even_gated(x: torch.Tensor, eps: float, stats: torch.Tensor, weight: torch.Tensor,
                       swiglu: "bool | str" = True) -> torch.Tensor:
-    """:func:`linear_scaled`'s gated form for at most 128 rows, by the kernel that deals the columns out evenly over the
+    """:func:`linear_scaled`'s gated form for at most 192 rows, by the kernel that deals the columns out evenly over the
     compute units: act(s g) * (s u) -> bfloat16 [M, I], weight [2 I, K] with gate and up rows interleaved in blocks of 16."""
     m, n, k = _even_operands(x, weight)
     if n % 32:

@@ -764,7 +764,8 @@ def test_product_into_the_stream_of_65_to_128_rows(m, n, k):
 
 @pytest.mark.parametrize("m, n, k, act", [(17, 32, 8, "silu"), (1, 96, 72, "silu"), (33, 24576, 64, "gelu_tanh"), (64, 27648 - 32, 136, "silu"),
                                           (32, 37888, 328, "silu"), (65, 37888 + 32, 72, "silu"), (128, 36864, 256, "gelu_tanh"),
-                                          (50, 160, 2048, "silu"), (128, 24576 + 64, 4096, "silu")])
+                                          (50, 160, 2048, "silu"), (128, 24576 + 64, 4096, "silu"),
+                                          (129, 37888 - 32, 200, "silu"), (192, 27648, 64, "gelu_tanh"), (177, 64, 2048, "silu")])
 def test_gated_product_with_its_columns_dealt_out_evenly(m, n, k, act):
     """Each number of strips and of row tiles, columns and K that end inside a workgroup and a stage, and rows 4 KB apart (whose
     workgroups start at different stages) against the float32 formula."""

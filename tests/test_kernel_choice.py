@@ -183,8 +183,10 @@ def test_even_shares_of_columns(monkeypatch):
     for n, k in ((16, 8), (130, 264), (8192, 8192), (3584, 18944), (1000, 70000)):    # every split has a stage
         count, stages = shape(64, n, k)[1], (k + 63) // 64
         assert count >= 1 and (count - 1) * ((stages + count - 1) // count) < stages
-    assert products.even_gated(17, 37888, 3584) and products.even_gated(128, 17920, 1536)
-    assert not any(products.even_gated(m, 37888, 3584) for m in (1, 16, 129)) and not products.even_gated(64, 9728, 896)
+    assert all(products.even_gated(m, 37888, 3584) for m in (17, 64, 128, 192)) and products.even_gated(128, 17920, 1536)
+    assert not any(products.even_gated(m, 37888, 3584) for m in (1, 16, 193)) and not products.even_gated(64, 9728, 896)
+    assert not products.even_gated(64, 16384, 3072) and not products.even_gated(129, 27648, 5120)
+    assert products.even_gated(64, 57344, 8192) and not products.even_gated(65, 57344, 8192) and not products.even_gated(64, 55296, 5120)
     assert products.even_residual(49, 3584, 18944) and not products.even_residual(48, 3584, 18944)
     assert not products.even_residual(64, 1536, 8960) and products.even_residual(128, 1536, 8960)
     assert not products.even_residual(129, 3584, 18944) and not products.even_residual(128, 3584, 3584)
