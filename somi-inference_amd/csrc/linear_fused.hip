@@ -50,12 +50,12 @@ struct FusedRope {
     int act;                  // the gated form's activation: 0 or 1 SiLU, 2 the tanh form of GELU
 };
 
-template <int MT, int NS, int MODE, typename TO, bool SWIGLU, bool TAIL, bool ROPE = false>
+template <int MT, int NS, int MODE, typename TO, bool SWIGLU, bool TAIL, bool ROPE = false, bool BLOCKS = false>
 __global__ void __launch_bounds__(FUSED_MAX_WAVES * 64)
 linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ bias,
                     TO* __restrict__ out, float* __restrict__ h, const float* __restrict__ norm_w, float eps,
                     const float* __restrict__ stats_in, int stats_blocks, int stats_stride,
-                    float* __restrict__ stats_out, bf16* __restrict__ xnext, int M, int N, int K, int row_blocks,
+                    float* __restrict__ stats_out, bf16* __restrict__ xnext, int M, int N, int K, int blocks_of_rows,
                     int column_blocks, FusedRope rope) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ float row_scale[64];
@@ -67,6 +67,8 @@ linear_fused_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, cons
     constexpr int NL = (NS + MT) * 2;              // loads per lane and chunk: 8 lanes read the 128 bytes of a row
     constexpr int TILES = NS * MT;
 
+    // (A kernel of its own for several blocks: what they need cost a single one of 8 rows 0.2 us.)
+    const int row_blocks = BLOCKS ? blocks_of_rows : 1;
     // More rows than a workgroup takes are blocks.  The blocks of a column block are eight workgroups apart, so they run on one die side by side
     // and the second finds w in that die's L2.
     int column_block = blockIdx.x, row0 = 0;
@@ -431,8 +433,8 @@ static int fused_waves(int mt, int strips, int workgroups, int K) {
     return waves;
 }
 
-template <int MT, int NS, int MODE, typename TO, bool SW, bool TL, bool ROPE>
-static void fused_launch_kernel(const void* x, const void* w, const float* bias, void* out, float* h,
+template <int MT, int NS, int MODE, typename TO, bool SW, bool TL, bool ROPE, bool BLOCKS>
+static void fused_launch_blocks(const void* x, const void* w, const float* bias, void* out, float* h,
                                 const float* norm_w, float eps, const float* stats_in, int stats_blocks,
                                 int stats_stride, float* stats_out, void* xnext, int M, int N, int K,
                                 const FusedRope& rope, hipStream_t stream) {
@@ -441,12 +443,22 @@ static void fused_launch_kernel(const void* x, const void* w, const float* bias,
     const dim3 grid(row_blocks > 1 ? ceil_div(column_blocks, 8) * 8 * row_blocks : column_blocks), block(waves * 64);
     const size_t smem = fused_lds(MT, NS, waves);
     if (smem > 64 * 1024)                            // beyond the default limit of dynamic LDS
-        (void)hipFuncSetAttribute((const void*)linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE>,
+        (void)hipFuncSetAttribute((const void*)linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE, BLOCKS>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    hipLaunchKernelGGL((linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE>), grid, block, smem, stream,
+    hipLaunchKernelGGL((linear_fused_kernel<MT, NS, MODE, TO, SW, TL, ROPE, BLOCKS>), grid, block, smem, stream,
                        (const bf16*)x, (const bf16*)w, bias, (TO*)out, h, norm_w, eps, stats_in, stats_blocks,
                        stats_stride > 0 ? stats_stride : 16 * ceil_div(M, 16), stats_out, (bf16*)xnext, M, N, K, row_blocks,
                        column_blocks, rope);
+}
+
+template <int MT, int NS, int MODE, typename TO, bool SW, bool TL, bool ROPE>
+static void fused_launch_kernel(const void* x, const void* w, const float* bias, void* out, float* h,
+                                const float* norm_w, float eps, const float* stats_in, int stats_blocks,
+                                int stats_stride, float* stats_out, void* xnext, int M, int N, int K,
+                                const FusedRope& rope, hipStream_t stream) {
+    const auto launch = M > 16 * MT ? fused_launch_blocks<MT, NS, MODE, TO, SW, TL, ROPE, true>
+                                    : fused_launch_blocks<MT, NS, MODE, TO, SW, TL, ROPE, false>;
+    launch(x, w, bias, out, h, norm_w, eps, stats_in, stats_blocks, stats_stride, stats_out, xnext, M, N, K, rope, stream);
 }
 
 // Row tiles (of 16) of a workgroup: four, or as many as there are; two or one where the blocks of 32 or 16 rows still find a compute

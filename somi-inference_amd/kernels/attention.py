@@ -51,6 +51,9 @@ def forms_supported(k_cache: torch.Tensor, block_table: torch.Tensor) -> bool:
     return bool(ops.library().somi_attention_bias_supported(k_cache.shape[3], k_cache.shape[2], block_table.shape[1]))
 
 
+F32_MOST_ENTRIES = 65535      # the float32 matrix-core kernel's grid has the requests in its third dimension
+
+
 def paged_attention(qkv: torch.Tensor, num_heads: int, k_cache: torch.Tensor, v_cache: torch.Tensor,
                     block_table: torch.Tensor, step, *, window: int, scale: float,
                     bias: torch.Tensor | None = None, score: "ops.ScoreShape | None" = None) -> torch.Tensor:
@@ -63,7 +66,8 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, k_cache: torch.Tensor, v_
     """
     if score is not None and not score.any:
         score = None
-    if bias is None and score is None and ops.attention_f32_supported(qkv, k_cache):
+    if (bias is None and score is None and step.entry_start.shape[0] <= F32_MOST_ENTRIES
+            and ops.attention_f32_supported(qkv, k_cache)):
         return ops.attention_f32(qkv, k_cache, v_cache, block_table, step.entry_start, step.entry_first_position,
                                  step.positions, step.max_entry_len, step.max_context, num_heads, window, scale)
     if not mfma_attention_supported(qkv, k_cache) or ((bias is not None or score is not None)
